@@ -88,15 +88,16 @@ struct RegionBuilder {
   SmallVec<Region, 8> v;  // the lists of one patch fit inline
   int nblk = 0;
   long items = 0;
-  void add(int patch, const HBox& b) {
+  void add(int patch, const HBox& b, int blk = kBlk, int dir = 0) {
     long cells = b.size();
     if (cells <= 0) return;
     items += cells;
     Region r;
     r.patch = patch;
+    r.dir = dir;
     for (int d = 0; d < 3; ++d) { r.lo[d] = b.lo[d]; r.n[d] = (int)b.n(d); }
     r.blk0 = nblk;
-    nblk += (int)((cells + kBlk - 1) / kBlk);
+    nblk += (int)((cells + blk - 1) / blk);
     v.push_back(r);
   }
   // a region of a tile kernel: one block per tx x ty column tile and
@@ -107,10 +108,23 @@ struct RegionBuilder {
     items += cells;
     Region r;
     r.patch = patch;
+    r.dir = 0;
     for (int d = 0; d < 3; ++d) { r.lo[d] = b.lo[d]; r.n[d] = (int)b.n(d); }
     r.blk0 = nblk;
     nblk += (int)(((b.n(0) + tx - 1) / tx) * ((b.n(1) + ty - 1) / ty) * ((b.n(2) + tz - 1) / tz));
     v.push_back(r);
+  }
+};
+
+// A face list under construction: the regions direction by direction, and
+// where each direction ends.
+struct FaceBuilder : RegionBuilder {
+  FaceList f{};
+  void end_dir(int d) {
+    long before = 0;
+    for (int e = 0; e < d; ++e) before += f.items[e];
+    f.items[d] = items - before;
+    for (int e = d + 1; e < 4; ++e) { f.reg[e] = (int)v.size(); f.blk[e] = nblk; }
   }
 };
 
@@ -402,31 +416,40 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
   }
   // region lists; faces on a physical boundary go to their own list
   const PatchIn* pin = in;
-  RegionBuilder st1_prim, st1_flux[3], st1_fbc[3], st1_upd, st2_prim, st2_flux[3],
-      st2_fbc[3], st2_upd, st1_sum, st2_sum;
+  RegionBuilder st1_prim, st1_upd, st2_prim, st2_upd, st1_sum, st2_sum;
+  FaceBuilder st1_flux, st1_fbc, st2_flux, st2_fbc;
   auto add_faces = [&](RegionBuilder& in, RegionBuilder& bc, int q, HBox f, int d) {
     const Consts& Cq = Ct[pin[q].cidx];
     if (Cq.phys[d]) {
       if (f.lo[d] == Cq.dom_lo[d]) {
         HBox b = f;
         b.hi[d] = b.lo[d];
-        bc.add(q, b);
+        bc.add(q, b, kBcBlock, d);
         f.lo[d] += 1;
       }
       if (f.hi[d] == Cq.dom_hi[d] + 1 && f.hi[d] >= f.lo[d]) {
         HBox b = f;
         b.lo[d] = b.hi[d];
-        bc.add(q, b);
+        bc.add(q, b, kBcBlock, d);
         f.hi[d] -= 1;
       }
     }
-    if (f.hi[d] >= f.lo[d]) in.add(q, f);
+    if (f.hi[d] >= f.lo[d]) in.add(q, f, kBlk, d);
   };
+  for (int d = 0; d < dims; ++d) {
+    for (int q = 0; q < n; ++q) {
+      if (rk2) add_faces(st1_flux, st1_fbc, q, G[q].fb[d], d);
+      HBox f = G[q].vb2;
+      f.hi[d] += 1;
+      add_faces(st2_flux, st2_fbc, q, f, d);
+    }
+    st1_flux.end_dir(d); st1_fbc.end_dir(d);
+    st2_flux.end_dir(d); st2_fbc.end_dir(d);
+  }
   for (int q = 0; q < n; ++q) {
     const PatchGeo& g = G[q];
     if (rk2) {
       st1_prim.add(q, grow(g.vb1, 2, dims));
-      for (int d = 0; d < dims; ++d) add_faces(st1_flux[d], st1_fbc[d], q, g.fb[d], d);
       if (fused) st1_upd.add_tiles(q, g.vb1, tz);
       else st1_upd.add(q, g.vb1);
       if (summed) st1_sum.add_tiles(q, g.vb1, tz, kSumTX, kSumTY);
@@ -474,21 +497,15 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
     } else {
       st2_prim.add(q, grow(g.vb2, 2, dims));
     }
-    for (int d = 0; d < dims; ++d) {
-      HBox f = g.vb2;
-      f.hi[d] += 1;
-      add_faces(st2_flux[d], st2_fbc[d], q, f, d);
-    }
     if (fused) st2_upd.add_tiles(q, g.vb2, tz);
     else st2_upd.add(q, g.vb2);
     if (summed) st2_sum.add_tiles(q, g.vb2, tz, kSumTX, kSumTY);
   }
-  constexpr int kLists = 18;
-  RegionBuilder* lists[kLists] = {&st1_prim, &st1_flux[0], &st1_flux[1], &st1_flux[2],
-                                  &st1_fbc[0], &st1_fbc[1], &st1_fbc[2], &st1_upd,
-                                  &st2_prim, &st2_flux[0], &st2_flux[1], &st2_flux[2],
-                                  &st2_fbc[0], &st2_fbc[1], &st2_fbc[2], &st2_upd,
-                                  &st1_sum, &st2_sum};
+  // stage 1's lists, then stage 2's (in the order of kPrim .. kSum)
+  enum { kPrim, kFlux, kFbc, kUpd, kSum, kStageLists };
+  constexpr int kLists = 2 * kStageLists;
+  RegionBuilder* lists[kLists] = {&st1_prim, &st1_flux, &st1_fbc, &st1_upd, &st1_sum,
+                                  &st2_prim, &st2_flux, &st2_fbc, &st2_upd, &st2_sum};
   // table layout inside the arena (after the scratch)
   // fused RK2: a second patch table for stage 2, whose W is the W of U*
   // that stage 1 wrote (the kernels always read W through the table)
@@ -622,16 +639,19 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
   double* dtp = reinterpret_cast<double*>(A + off_dtp);
   long* idp = reinterpret_cast<long*>(A + off_idp);
   const Consts* ct = reinterpret_cast<const Consts*>(A + off_ct);
-  auto stage = [&](int l0) {
+  auto fl = [&](int l) {
+    FaceList f = static_cast<FaceBuilder*>(lists[l])->f;
+    f.r = reinterpret_cast<const Region*>(A + off_reg[l]);
+    return f;
+  };
+  auto stage = [&](int st) {
+    const int l0 = st * kStageLists;
     StageLists L;
-    L.prim = rl(l0);
-    for (int d = 0; d < 3; ++d) {
-      L.flux[d] = rl(l0 + 1 + d);
-      L.fbc[d] = rl(l0 + 4 + d);
-      if (d >= dims) { L.flux[d].nblk = 0; L.fbc[d].nblk = 0; }
-    }
-    L.upd = rl(l0 + 7);
-    L.sum = rl(l0 == 0 ? 16 : 17);
+    L.prim = rl(l0 + kPrim);
+    L.flux = fl(l0 + kFlux);
+    L.fbc = fl(l0 + kFbc);
+    L.upd = rl(l0 + kUpd);
+    L.sum = rl(l0 + kSum);
     L.fused = fused ? 1 : 0;
     L.summed = summed ? 1 : 0;
     return L;
@@ -664,7 +684,7 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
       if (e2 != hipSuccess) return hipfail(c, e2, "predictor launch");
       if (c->timer) n_stage1 = c->timer->n;
       StepArgs S2{1.0, 1, 0, 0, 0, 2, 1, 0, c->walk_tile, c->walk_xcd, 2, tz};
-      e2 = launch(stage(8), S2);
+      e2 = launch(stage(1), S2);
       if (e2 != hipSuccess) return hipfail(c, e2, "corrector launch");
     } else if (rk2) {
       StepArgs S1{1.0, 0, 0, 1, 0, 0, 0, 1, c->walk_tile, c->walk_xcd, 0, tz};
@@ -672,14 +692,14 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
       if (e2 != hipSuccess) return hipfail(c, e2, "stage 1 launch");
       if (c->timer) n_stage1 = c->timer->n;
       StepArgs S2{0.5, 1, 1, 0, 1, 1, 1, 0, c->walk_tile, c->walk_xcd, 0, tz};
-      e2 = launch(stage(8), S2);
+      e2 = launch(stage(1), S2);
       if (e2 != hipSuccess) return hipfail(c, e2, "stage 2 launch");
     } else {
       StepArgs S{1.0, 0, 0, 0, 0, 2, 1, 0, c->walk_tile, c->walk_xcd, 0, tz};
-      e2 = launch(stage(8), S);
+      e2 = launch(stage(1), S);
       if (e2 != hipSuccess) return hipfail(c, e2, "first-order launch");
     }
-    RegionList U2 = rl(15);
+    RegionList U2 = rl(kStageLists + kUpd);
     e2 = launch_dt_final(U2, dtp, idp, reinterpret_cast<double*>(A + off_dto),
                          reinterpret_cast<long*>(A + off_ido), st);
     if (e2 != hipSuccess) return hipfail(c, e2, "dt reduction launch");

@@ -200,6 +200,37 @@ __device__ __forceinline__ void limit(int lim, T wl, T w0, T wr, T& left,
   }
 }
 
+// ----------------------------------------------------------- face frame --
+// The frame of a face of direction d: the normal and the two tangential
+// directions as velocity component numbers.  Face arithmetic runs in this
+// frame (rho, un, ut1, ut2, p, bn, bt1, bt2, then psi); the rotation is the
+// choice of the components to load and store, whose addresses are scalar, so
+// one body serves the three directions with d taken at run time.
+struct Frame {
+  int d, n, t1, t2;
+  __device__ __forceinline__ explicit Frame(int dir)
+      : d(dir), n(1 + dir), t1(dir == 2 ? 1 : dir + 2), t2(dir == 0 ? 3 : dir) {}
+  // component number of frame entry q (0..8) of the plasma
+  __device__ __forceinline__ int plasma(int q) const {
+    return q == 1 ? n : q == 2 ? t1 : q == 3 ? t2
+         : q == 5 ? 4 + n : q == 6 ? 4 + t1 : q == 7 ? 4 + t2 : q;
+  }
+  // offset of frame entry q (0..4) in a neutral fluid's components
+  __device__ __forceinline__ int neutral(int q) const {
+    return q == 1 ? n : q == 2 ? t1 : q == 3 ? t2 : q;
+  }
+  // the limiter of plasma entry q (a scalar select between constant-offset
+  // loads: a byte load at a run-time offset would not be scalar)
+  __device__ __forceinline__ int limiter(const Consts& C, int q) const {
+    auto pick = [](int v, int a, int b, int c) { return v == 1 ? a : v == 2 ? b : c; };
+    if (q >= 1 && q <= 3)
+      return pick(plasma(q), C.lim[1], C.lim[2], C.lim[3]);
+    if (q >= 5 && q <= 7)
+      return pick(plasma(q) - 4, C.lim[5], C.lim[6], C.lim[7]);
+    return C.lim[q];
+  }
+};
+
 // ----------------------------------------- characteristic reconstruction --
 // *FACESLOPES (src/reconstructionF.ChF): limited slopes SL (lo side) and SR
 // (hi side) of a cell from its one-sided differences dSL = W - W(i-1),
@@ -331,8 +362,8 @@ __device__ __forceinline__ T tvd_hi(T wp, T w0, T dWL, T dWR) {
   return w0 + minmod3(dWL, dWR, wp - w0);
 }
 
-// Eigen-structure of the ideal-MHD system at one cell along dir, formed from
-// the cell's primitive state as in CHARANALYSISF / CHARSYNTHESISF
+// Eigen-structure of the ideal-MHD system at one cell along the normal of
+// the face frame, formed from the cell's primitive state as in CHARANALYSISF / CHARSYNTHESISF
 // (srcIdeal/PatchIdealMHDF.ChF:1167-1505).  The fast / slow weights take the
 // degenerate branch below 1e-12 in the analysis (aF, aS) and below 1e-8 in
 // the synthesis (aF2, aS2).
@@ -349,9 +380,9 @@ __device__ __forceinline__ void char_alpha(T dfs, T cc, T aas, T aaf, T eps, T& 
   else { aF = tsqrt((cc - aas) / dfs); aS = tsqrt((aaf - cc) / dfs); }
 }
 
-template <typename T, int dir>
+template <typename T>
 __device__ __forceinline__ CharBasis<T> char_basis(const Consts& C, const T* w) {
-  constexpr int bn = 5 + dir, bt1 = 5 + (dir + 1) % 3, bt2 = 5 + (dir + 2) % 3;
+  constexpr int bn = 5, bt1 = 6, bt2 = 7;
   CharBasis<T> B;
   const T PGas = fmaxr((T)C.smallp, w[4]);
   const T Rho = fmaxr((T)C.smallr, w[0]);
@@ -388,12 +419,11 @@ __device__ __forceinline__ CharBasis<T> char_basis(const Consts& C, const T* w) 
 }
 
 // CHARANALYSISF (:1252-1325): primitive differences d (plasma components in
-// Cartesian order) -> characteristic variables a (entropy, div(B), two
+// the face frame) -> characteristic variables a (entropy, div(B), two
 // Alfven, two fast, two slow).
-template <typename T, int dir>
+template <typename T>
 __device__ __forceinline__ void char_analysis(const CharBasis<T>& B, const T* d, T* a) {
-  constexpr int n = 1 + dir, t1 = 1 + (dir + 1) % 3, t2 = 1 + (dir + 2) % 3;
-  constexpr int bn = 5 + dir, bt1 = 5 + (dir + 1) % 3, bt2 = 5 + (dir + 2) % 3;
+  constexpr int n = 1, t1 = 2, t2 = 3, bn = 5, bt1 = 6, bt2 = 7;
   // SIGN(one, BX) with -0.0 counted as positive, as the synthesis's BX < 0
   // test does, so that both transforms agree where the field is exactly zero
   const T two = T(2), siBX = B.BX < T(0) ? T(-1) : T(1);
@@ -418,10 +448,9 @@ __device__ __forceinline__ void char_analysis(const CharBasis<T>& B, const T* d,
 
 // CHARSYNTHESISF (:1438-1502): characteristic variables -> primitive
 // differences.
-template <typename T, int dir>
+template <typename T>
 __device__ __forceinline__ void char_synthesis(const CharBasis<T>& B, const T* a, T* d) {
-  constexpr int n = 1 + dir, t1 = 1 + (dir + 1) % 3, t2 = 1 + (dir + 2) % 3;
-  constexpr int bn = 5 + dir, bt1 = 5 + (dir + 1) % 3, bt2 = 5 + (dir + 2) % 3;
+  constexpr int n = 1, t1 = 2, t2 = 3, bn = 5, bt1 = 6, bt2 = 7;
   const T betaYX = B.BX < T(0) ? -B.betaY : B.betaY;
   const T betaZX = B.BX < T(0) ? -B.betaZ : B.betaZ;
   const T alpha3 = T(kSQRT_2) * a[2], alpha4 = T(kSQRT_2) * a[3];

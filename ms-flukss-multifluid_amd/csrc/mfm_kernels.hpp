@@ -38,12 +38,14 @@ struct DevPatch {
   double psi_decay[2];   // exp(-dt_stage Ch^2/Cp^2) of stage 0 / 1
 };
 
-// A box of work items belonging to one patch; blk0 = first block.
+// A box of work items belonging to one patch; blk0 = first block; dir: the
+// direction of the faces of a face list.
 struct Region {
   int patch;
   int lo[3];
   int n[3];
   int blk0;
+  int dir;
 };
 
 struct RegionList {
@@ -53,14 +55,32 @@ struct RegionList {
   long items;       // cells (or faces) covered
 };
 
-// flux[d]: interior faces of direction d; fbc[d]: faces of direction d on
-// a physical (non-periodic) domain boundary.
+// The faces of every direction in one list, the regions of direction d at
+// [reg[d], reg[d + 1]) with the blocks [blk[d], blk[d + 1]).
+struct FaceList {
+  const Region* r;  // device pointer
+  int reg[4];
+  int blk[4];
+  long items[3];
+};
+
+// The part of a FaceList that a launch covers: nreg regions from r on, the
+// blocks from blk[0] on, direction by direction (blk[q] .. blk[q + 1]).
+struct FaceBlocks {
+  int nreg;
+  int blk[4];
+};
+
+// flux: interior faces; fbc: faces on a physical (non-periodic) domain
+// boundary (in blocks of kBcBlock).
+constexpr int kBcBlock = 64;
 struct StageLists {
-  RegionList prim, flux[3], fbc[3], upd, sum;
+  RegionList prim, upd, sum;
+  FaceList flux, fbc;
   int fused;        // upd is a list of k_stage tiles (interior faces and the
-                    // update in one launch); flux[] is then unused
+                    // update in one launch); flux is then unused
   int summed;       // sum is a list of tiles whose face sums (D) the face-sum
-                    // kernels form; k_update then reads D; flux[] unused
+                    // kernels form; k_update then reads D; flux unused
 };
 
 struct StepArgs {
