@@ -9,62 +9,77 @@
 namespace mfm {
 namespace {
 constexpr int kFB = 256;
+// Components per thread: blockIdx.y takes a chunk of the components, so that
+// the few thousand cells of a small level still fill the chip and a thread
+// keeps one batch of independent loads in flight.
+constexpr int kCopyComps = 8, kInterpComps = 4;
+
+// Blocks are dispatched round-robin over the 8 XCDs, each with its own L2:
+// give every XCD one contiguous range of blocks, hence of boxes.  The ghost
+// rows of a box are 4 cells wide in x, and a row's right ghost and the next
+// row's left ghost share a cache line; written from one XCD they meet in its
+// L2 and leave as one line.  With the component
+// chunks: the fill of two levels of 343 boxes of 16^3 cells (4 ghosts, 23
+// components; two exchanges, one interpolation) 0.99 -> 0.90 ms.
+__device__ __forceinline__ int xcd_block() {
+  const int nb = (int)gridDim.x, b = (int)blockIdx.x;
+  const int q = nb >> 3, r = nb & 7, x = b & 7;
+  return x * q + (x < r ? x : r) + (b >> 3);
+}
 
 __device__ __forceinline__ long fab_off(const FillFab& F, int i, int j, int k) {
   return (long)(i - F.lo[0]) +
          (long)F.n[0] * ((long)(j - F.lo[1]) + (long)F.n[1] * (long)(k - F.lo[2]));
 }
 
-// Copy of the nc components of one cell, in batches of 8 loads issued
-// before their stores so that every lane keeps several loads in flight.
+// Copy of the components c0 .. c0 + kCopyComps - 1 (below nc) of one cell, the
+// loads issued before the stores so that every lane keeps them in flight.
 // mode 0: dst = new; 1: dst = old; 2: dst = new*a + old*b (b = 1 - a), the
 // order of timeInterp (srcIdeal/PiecewiseLinearFillPatchMHDAM.cpp:489-496).
 __device__ __forceinline__ void copy_cell(double* dp, long dcs, const double* sp,
                                           long scs, const double* op, long ocs,
-                                          int nc, double a, double b, int mode) {
-  constexpr int kBatch = 8;
-  double v[kBatch], w[kBatch];
-  for (int c0 = 0; c0 < nc; c0 += kBatch) {
-    const int m = nc - c0 < kBatch ? nc - c0 : kBatch;
+                                          int c0, int nc, double a, double b, int mode) {
+  double v[kCopyComps], w[kCopyComps];
+  const int m = nc - c0 < kCopyComps ? nc - c0 : kCopyComps;
 #pragma unroll
-    for (int q = 0; q < kBatch; ++q)
-      if (q < m) v[q] = (mode == 1 ? op[(c0 + q) * ocs] : sp[(c0 + q) * scs]);
-    if (mode == 2) {
+  for (int q = 0; q < kCopyComps; ++q)
+    if (q < m) v[q] = (mode == 1 ? op[(c0 + q) * ocs] : sp[(c0 + q) * scs]);
+  if (mode == 2) {
 #pragma unroll
-      for (int q = 0; q < kBatch; ++q)
-        if (q < m) w[q] = op[(c0 + q) * ocs];
+    for (int q = 0; q < kCopyComps; ++q)
+      if (q < m) w[q] = op[(c0 + q) * ocs];
 #pragma unroll
-      for (int q = 0; q < kBatch; ++q)
-        if (q < m) {
-          const double x = v[q] * a;
-          const double y = w[q] * b;
-          v[q] = x + y;
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < kBatch; ++q)
-      if (q < m) dp[(c0 + q) * dcs] = v[q];
+    for (int q = 0; q < kCopyComps; ++q)
+      if (q < m) {
+        const double x = v[q] * a;
+        const double y = w[q] * b;
+        v[q] = x + y;
+      }
   }
+#pragma unroll
+  for (int q = 0; q < kCopyComps; ++q)
+    if (q < m) dp[(c0 + q) * dcs] = v[q];
 }
 
 __global__ __launch_bounds__(kFB) void k_rect_copy(
     const CopyRect* __restrict__ R, int nr, const FillFab* __restrict__ Sn,
     const FillFab* __restrict__ So, const FillFab* __restrict__ D, int nc,
     double a, double b, int mode) {
-  const int bx = blockIdx.x;
+  const int bx = xcd_block();
   int lo = 0, hi = nr - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
     if (R[mid].blk0 <= bx) lo = mid; else hi = mid - 1;
   }
   const CopyRect r = R[lo];
-  const long t = (long)(bx - r.blk0) * kFB + threadIdx.x;
-  const long n01 = (long)r.n[0] * r.n[1];
+  // (2^32 cells of one component would be 34 GB)
+  const unsigned t = (unsigned)(bx - r.blk0) * kFB + threadIdx.x;
+  const unsigned n01 = (unsigned)r.n[0] * r.n[1];
   if (t >= n01 * r.n[2]) return;
   const int k = (int)(t / n01);
-  const long rem = t - (long)k * n01;
-  const int j = (int)(rem / r.n[0]);
-  const int i = (int)(rem - (long)j * r.n[0]);
+  const unsigned rem = t - (unsigned)k * n01;
+  const int j = (int)(rem / (unsigned)r.n[0]);
+  const int i = (int)(rem - (unsigned)j * r.n[0]);
   const FillFab d = D[r.dst];
   double* dp = d.p + fab_off(d, r.dlo[0] + i, r.dlo[1] + j, r.dlo[2] + k);
   const int si = r.slo[0] + i, sj = r.slo[1] + j, sk = r.slo[2] + k;
@@ -73,7 +88,7 @@ __global__ __launch_bounds__(kFB) void k_rect_copy(
   long scs = 0, ocs = 0;
   if (mode != 1) { const FillFab s = Sn[r.src]; sp = s.p + fab_off(s, si, sj, sk); scs = s.cs; }
   if (mode != 0) { const FillFab o = So[r.src]; op = o.p + fab_off(o, si, sj, sk); ocs = o.cs; }
-  copy_cell(dp, d.cs, sp, scs, op, ocs, nc, a, b, mode);
+  copy_cell(dp, d.cs, sp, scs, op, ocs, (int)blockIdx.y * kCopyComps, nc, a, b, mode);
 }
 
 // The same three modes for a list of single cells (the coarse cells the
@@ -82,7 +97,7 @@ __global__ __launch_bounds__(kFB) void k_cell_copy(
     const GatherCell* __restrict__ G, long n, const FillFab* __restrict__ Sn,
     const FillFab* __restrict__ So, const FillFab* __restrict__ D, int nc,
     double a, double b, int mode) {
-  const long t = (long)blockIdx.x * kFB + threadIdx.x;
+  const long t = (long)xcd_block() * kFB + threadIdx.x;
   if (t >= n) return;
   const GatherCell g = G[t];
   const FillFab d = D[g.dst];
@@ -91,7 +106,7 @@ __global__ __launch_bounds__(kFB) void k_cell_copy(
   long scs = 0, ocs = 0;
   if (mode != 1) { const FillFab s = Sn[g.src]; sp = s.p + fab_off(s, g.s[0], g.s[1], g.s[2]); scs = s.cs; }
   if (mode != 0) { const FillFab o = So[g.src]; op = o.p + fab_off(o, g.s[0], g.s[1], g.s[2]); ocs = o.cs; }
-  copy_cell(d.p + g.doff, d.cs, sp, scs, op, ocs, nc, a, b, mode);
+  copy_cell(d.p + g.doff, d.cs, sp, scs, op, ocs, (int)blockIdx.y * kCopyComps, nc, a, b, mode);
 }
 
 // minmod of src/reconstructionF.ChF:4-14: sign(1,A) max(0, min(|A|, sign(1,A) B))
@@ -223,7 +238,7 @@ __device__ __forceinline__ void write_children(const InterpArgs& A,
 }
 
 __global__ __launch_bounds__(kFB) void k_fill_interp(InterpArgs A) {
-  const long t = (long)blockIdx.x * kFB + threadIdx.x;
+  const long t = (long)xcd_block() * kFB + threadIdx.x;
   if (t >= A.ncell) return;
   const int2 e = A.cell[t];
   const FillPatch P = A.P[e.x];
@@ -248,13 +263,14 @@ __global__ __launch_bounds__(kFB) void k_fill_interp(InterpArgs A) {
   X.st[0] = 1; X.st[1] = P.wn[0]; X.st[2] = n01;
   X.dims = A.dims;
   X.fl = A.flag[t];
-  for (int c = 0; c < A.nc; ++c) {
+  const int c0 = (int)blockIdx.y * kInterpComps, c1 = min(c0 + kInterpComps, A.nc);
+  for (int c = c0; c < c1; ++c) {
     if (A.ibx >= 0 && c >= A.ibx && c < A.ibx + A.dims) continue;
     double s[3];
     const double w0 = slopes(X, A, c, s);
     write_children(A, F, f0, f1, ci, c, w0, s);
   }
-  if (A.ibx >= 0) {
+  if (A.ibx >= c0 && A.ibx < c1) {  // the chunk that holds the first of B
     // the slopes of B_d along d are corrected together, then each component
     // is written with its own three slopes
     double sb[3][3], wb[3];
@@ -268,6 +284,7 @@ __global__ __launch_bounds__(kFB) void k_fill_interp(InterpArgs A) {
       write_children(A, F, f0, f1, ci, A.ibx + q, wb[q], sb[q]);
   }
 }
+unsigned comp_blocks(int nc, int per) { return (unsigned)((nc + per - 1) / per); }
 }  // namespace
 
 hipError_t launch_rect_copy(const CopyRect* R, int nr, int nblk,
@@ -275,7 +292,7 @@ hipError_t launch_rect_copy(const CopyRect* R, int nr, int nblk,
                             const FillFab* dst, int nc, double a, double b,
                             int mode, hipStream_t s) {
   if (nr <= 0 || nblk <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_rect_copy, dim3((unsigned)nblk), dim3(kFB), 0, s, R, nr,
+  hipLaunchKernelGGL(k_rect_copy, dim3((unsigned)nblk, comp_blocks(nc, kCopyComps)), dim3(kFB), 0, s, R, nr,
                      src_new, src_old, dst, nc, a, b, mode);
   return hipGetLastError();
 }
@@ -284,14 +301,16 @@ hipError_t launch_cell_copy(const GatherCell* G, long n, const FillFab* src_new,
                             const FillFab* src_old, const FillFab* dst, int nc,
                             double a, double b, int mode, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_cell_copy, dim3((unsigned)((n + kFB - 1) / kFB)), dim3(kFB), 0, s,
-                     G, n, src_new, src_old, dst, nc, a, b, mode);
+  hipLaunchKernelGGL(k_cell_copy,
+                     dim3((unsigned)((n + kFB - 1) / kFB), comp_blocks(nc, kCopyComps)), dim3(kFB), 0,
+                     s, G, n, src_new, src_old, dst, nc, a, b, mode);
   return hipGetLastError();
 }
 
 hipError_t launch_fill_interp(const InterpArgs& A, hipStream_t s) {
   if (A.ncell <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fill_interp, dim3((unsigned)((A.ncell + kFB - 1) / kFB)),
+  hipLaunchKernelGGL(k_fill_interp,
+                     dim3((unsigned)((A.ncell + kFB - 1) / kFB), comp_blocks(A.nc, kInterpComps)),
                      dim3(kFB), 0, s, A);
   return hipGetLastError();
 }
