@@ -245,6 +245,7 @@ int build_consts(const mfm_params* p, Consts& C, std::string& why) {
   for (int c = 1; c < 8 + C.dedner; ++c)
     if (C.lim[c] != C.lim[0]) C.plasma_lim = -1;
   C.gamma = p->gamma;
+  C.invgamma = 1.0 / p->gamma;
   C.hgamma = p->gamma - 1.0;
   C.invhgamma = 1.0 / C.hgamma;
   C.smallr = p->smallr;
