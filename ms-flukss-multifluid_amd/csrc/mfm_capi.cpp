@@ -24,7 +24,24 @@ namespace mfm {
 namespace host {
 
 constexpr int kBlk = 256;
-constexpr double kAutoTileFill = 0.75;  // MFM_STAGE_AUTO: cells / tile slots
+// MFM_STAGE_AUTO.  FP32 fluxes: the face sums for a call whose cells fill this
+// part of their 64 x 8 tiles; else (and in FP64 and for Hancock's corrector)
+// from so many cells on, in 3-D, with one plasma limiter that has a kernel of
+// its own.  Per RK2 step, separate kernels against face sums: FP32, 4 fluids,
+// 80^3 481 / 468 us, 96^3 815 / 759, 128^3 1.82 / 1.67 ms, 192^3 5.87 / 5.11;
+// 2 fluids 96^3 536 / 456 us, 128^3 1.21 / 1.03 ms; 1 fluid 96^3 277 / 296 us, 128^3
+// 681 / 656; FP64, 4 fluids, 96^3 1.31 / 1.37 ms, 128^3 3.01 / 2.88, 160^3 5.80 / 5.40;
+// 2 fluids 128^3 1.83 / 1.84, 160^3 3.46 / 3.39, 1 fluid slower at every size (the
+// plasma tile kernel holds 2 wavefronts per SIMD, the face kernel 3; the
+// gain is the neutral fluids'); Hancock, FP32, 4 fluids 96^3 0.70 / 0.70, 128^3
+// 1.56 / 1.45 ms.
+constexpr double kAutoTileFill = 0.75;
+constexpr double kAutoCells = 6.0e5, kAutoCells1 = 2.0e6, kAutoCellsHan = 1.3e6,
+                 kAutoCells64 = 2.0e6;
+// Blocks of 512 threads (twice as many of 256) below which the z-chunks get
+// shorter: 64^3, FP32, 2 fluids, chunks of 8 / 4 / 2 / 1 planes 405 / 261 / 204 / 185 us;
+// 96^3 595 / 456 / 454 / 458; 128^3 1079 / 1028 / 1037 / 1080.
+constexpr double kAutoBlocks = 1000.0;
 const double eos_mp = 1.67262171e-24, eos_k = 1.3806505e-16;
 
 int fail(mfm_ctx* c, int code, const std::string& m) {
@@ -49,6 +66,7 @@ int ensure_arena(mfm_ctx* c, size_t bytes) {
   hipError_t e = hipMalloc((void**)&c->arena, want);
   if (e != hipSuccess) {
     c->arena = nullptr;
+    (void)hipGetLastError();  // a later launch check must not find this error
     return fail(c, MFM_ERR_NOMEM, "hipMalloc of scratch failed");
   }
   c->arena_bytes = want;
@@ -95,13 +113,14 @@ struct RegionBuilder {
     Region r;
     r.patch = patch;
     r.dir = dir;
+    r.tx = r.ty = r.tz = 0;
     for (int d = 0; d < 3; ++d) { r.lo[d] = b.lo[d]; r.n[d] = (int)b.n(d); }
     r.blk0 = nblk;
     nblk += (int)((cells + blk - 1) / blk);
     v.push_back(r);
   }
   // a region of a tile kernel: one block per tx x ty column tile and
-  // z-chunk of tz planes (k_stage: 16 x 16, k_fsum: 64 x 8)
+  // z-chunk of tz planes
   void add_tiles(int patch, const HBox& b, int tz, int tx = 16, int ty = 16) {
     long cells = b.size();
     if (cells <= 0) return;
@@ -109,10 +128,71 @@ struct RegionBuilder {
     Region r;
     r.patch = patch;
     r.dir = 0;
+    r.tx = tx;
+    r.ty = ty;
+    // chunks of one height as far as the box allows
+    const int nz = (int)b.n(2), chunks = (nz + tz - 1) / tz;
+    r.tz = tz = (nz + chunks - 1) / chunks;
     for (int d = 0; d < 3; ++d) { r.lo[d] = b.lo[d]; r.n[d] = (int)b.n(d); }
     r.blk0 = nblk;
-    nblk += (int)(((b.n(0) + tx - 1) / tx) * ((b.n(1) + ty - 1) / ty) * ((b.n(2) + tz - 1) / tz));
+    nblk += (int)(((b.n(0) + tx - 1) / tx) * ((b.n(1) + ty - 1) / ty) * ((nz + tz - 1) / tz));
     v.push_back(r);
+  }
+};
+
+// The tile of the face-sum kernels for a box of nx x ny columns.  A tile's
+// faces of one direction take whole wavefronts (issue) in whole rounds of the
+// block's threads (a barrier waits for the last): the shape with the smallest
+// sum of both over the box, the wider one on a tie.
+// TILE_MEASURED
+struct Tile { int tx, ty; };
+long tile_rounds(const Tile& t, int block) {
+  auto rounds = [&](long f) { return (f + block - 1) / block; };
+  return rounds((t.tx + 1L) * t.ty) + rounds(t.tx * (t.ty + 1L)) + rounds((long)t.tx * t.ty);
+}
+Tile sum_tile(long nx, long ny, int block, int slots) {
+  Tile best{1, 1};
+  long cost = std::numeric_limits<long>::max();
+  for (long kx = 1; kx == 1 || kx <= nx / 16; ++kx) {
+    const long tx = std::min((nx + kx - 1) / kx, (long)block);
+    const long most = std::min({(long)block / tx, (slots - tx) / (3 * tx + 1), ny});
+    for (long ty = most; ty >= 1 && 2 * ty > most; --ty) {
+      const Tile t{(int)tx, (int)ty};
+      const long pass = tile_rounds(t, 64) + tile_rounds(t, block) * (block / 64);
+      const long c = ((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) * pass;
+      if (c < cost) {
+        cost = c;
+        best = t;
+      }
+    }
+  }
+  return best;
+}
+
+// Adds the wavefront rounds a box's planes take in blocks of `block` threads
+// (a block holds its wavefronts' slots whether they have faces or not), and its
+// tile planes.
+void sum_rounds(const HBox& b, const Tile& t, int block, double& work, double& planes) {
+  const double np = (double)((b.n(0) + t.tx - 1) / t.tx * ((b.n(1) + t.ty - 1) / t.ty)) * (double)b.n(2);
+  planes += np;
+  work += np * (double)(tile_rounds(t, block) * (block / 64));
+}
+
+// The tiles of the boxes of one call, by their sizes (a level has few).
+struct TileCache {
+  int block, slots;
+  SmallVec<Region, 4> seen;  // n: columns; tx, ty: their tile
+  Tile of(const HBox& b) {
+    for (int q = 0; q < seen.size(); ++q)
+      if (seen[q].n[0] == b.n(0) && seen[q].n[1] == b.n(1)) return {seen[q].tx, seen[q].ty};
+    const Tile t = sum_tile(b.n(0), b.n(1), block, slots);
+    Region r{};
+    r.n[0] = (int)b.n(0);
+    r.n[1] = (int)b.n(1);
+    r.tx = t.tx;
+    r.ty = t.ty;
+    seen.push_back(r);
+    return t;
   }
 };
 
@@ -343,40 +423,56 @@ int check_patch(const Consts& C0, const Consts& Cq, int ng, const PatchIn& P, co
 // precision).  c provides the scratch arena, staging, timer and errors.
 int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
               double* new_dt, int* min_cell, double* level_dt, int* min_patch,
-              hipStream_t s, const FixedScratch* fixed) {
+              hipStream_t s, const FixedScratch* fixed, bool separate) {
   const Consts& C0 = Ct[0];
   const mfm_params& p = c->p;
   const int dims = C0.dims;
   const bool rk2 = p.time_approx == MFM_TIME_RK2;
   const bool han = p.time_approx == MFM_TIME_HANCOCK;
   const int ng = rk2 ? 4 : (han ? 3 : 2);  // PatchMHDAM::numGhostCells
-  // tile kernels for the interior faces (k_stage, or k_fsum before
-  // k_update); the Hancock scheme and characteristic slopes keep the
-  // separate kernels, and so does the FP64 build for the summed stages: it
-  // applies the directions one at a time, in the reference's order
-  int mode = (han || C0.char_rec) ? MFM_STAGE_SEPARATE : c->stage_mode;
-  if (mode == MFM_STAGE_AUTO) {
-    // the summed stages where their 64 x 8 column tiles are well filled
-    // (FP32-flux build; the allocation-free entry point keeps the separate
-    // kernels, whose scratch its bound is stated for)
+  // Tile kernels for the interior faces: k_stage, or the face sums before
+  // k_update (the Hancock corrector's too).  Characteristic slopes keep the
+  // separate kernels; so does the allocation-free entry point where it did
+  // before the face sums covered the case (its scratch bound is stated for
+  // the separate kernels).
+  const bool f32 = p.precision == MFM_PREC_FP32_FLUX;
+  int mode = c->stage_mode;
+  if (C0.char_rec || (han && mode == MFM_STAGE_FUSED) ||
+      (fixed && mode == MFM_STAGE_SUMMED && (han || !f32)))
     mode = MFM_STAGE_SEPARATE;
-    if (p.precision == MFM_PREC_FP32_FLUX && !fixed) {
-      double cells = 0.0, slots = 0.0;
+  const bool choose = mode == MFM_STAGE_AUTO;
+  int sum_block = f32 ? 512 : 256;
+  int tz = std::max(1, c->stage_tz);
+  const int slots256 = sum_slots(256, f32 ? 4 : 8, C0.dedner);
+  if (choose) {
+    mode = MFM_STAGE_SEPARATE;
+    if (!fixed && !separate) {
+      TileCache t512{512, sum_slots(512, 4, 0), {}}, t256{256, slots256, {}};
+      double cells = 0.0, slots = 0.0, r512 = 0.0, r256 = 0.0, p512 = 0.0, p256 = 0.0;
       for (int q = 0; q < n; ++q) {
         if (in[q].cidx < 0 || in[q].cidx >= nct) continue;
         const HBox v = clip(Ct[in[q].cidx], hb(in[q].valid));
         if (v.size() <= 0) continue;
         cells += (double)v.size();
-        slots += (double)((v.n(0) + kSumTX - 1) / kSumTX * kSumTX) *
-                 (double)((v.n(1) + kSumTY - 1) / kSumTY * kSumTY) * (double)v.n(2);
+        slots += (double)((v.n(0) + 63) / 64 * 64) * (double)((v.n(1) + 7) / 8 * 8) * (double)v.n(2);
+        if (f32) sum_rounds(v, t512.of(v), 512, r512, p512);
+        sum_rounds(v, t256.of(v), 256, r256, p256);
       }
-      if (slots > 0.0 && cells >= kAutoTileFill * slots) mode = MFM_STAGE_SUMMED;
+      if (f32 && !han && slots > 0.0 && cells >= kAutoTileFill * slots) mode = MFM_STAGE_SUMMED;
+      const bool one_lim = C0.plasma_lim == MFM_LIM_MINMOD || C0.plasma_lim == MFM_LIM_VANLEER;
+      const double least = f32 ? (han ? kAutoCellsHan : (C0.nf > 1 ? kAutoCells : kAutoCells1))
+                               : (C0.nf > 2 ? kAutoCells64 : 2.0 * kAutoCells64);
+      if (dims == 3 && one_lim && (C0.nf > 1 || (f32 && !han)) && cells >= least)
+        mode = MFM_STAGE_SUMMED;
+      if (f32 && r256 < r512) sum_block = 256;
+      // shorter z-chunks where the blocks would not fill the chip twice over
+      const double planes = sum_block == 512 ? p512 : 0.5 * p256;
+      while (tz > 1 && planes < kAutoBlocks * tz) tz /= 2;
     }
   }
-  if (mode == MFM_STAGE_SUMMED && p.precision != MFM_PREC_FP32_FLUX) mode = MFM_STAGE_SEPARATE;
+  TileCache tiles{sum_block, sum_block == 512 ? sum_slots(512, 4, 0) : slots256, {}};
   const bool fused = mode == MFM_STAGE_FUSED;
   const bool summed = mode == MFM_STAGE_SUMMED;
-  const int tz = std::max(1, c->stage_tz);
   if (n <= 0) return fail(c, MFM_ERR_ARG, "empty patch table");
   for (int r = 1; r < nct; ++r)
     if (Ct[r].dims != C0.dims || Ct[r].nf != C0.nf || Ct[r].dedner != C0.dedner)
@@ -437,6 +533,10 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
     }
     if (f.hi[d] >= f.lo[d]) in.add(q, f, kBlk, d);
   };
+  auto add_sum = [&](RegionBuilder& b, int q, const HBox& v) {
+    const Tile t = tiles.of(v);
+    b.add_tiles(q, v, tz, t.tx, t.ty);
+  };
   for (int d = 0; d < dims; ++d) {
     for (int q = 0; q < n; ++q) {
       if (rk2) add_faces(st1_flux, st1_fbc, q, G[q].fb[d], d);
@@ -453,7 +553,7 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
       st1_prim.add(q, grow(g.vb1, 2, dims));
       if (fused) st1_upd.add_tiles(q, g.vb1, tz);
       else st1_upd.add(q, g.vb1);
-      if (summed) st1_sum.add_tiles(q, g.vb1, tz, kSumTX, kSumTY);
+      if (summed) add_sum(st1_sum, q, g.vb1);
     } else if (han) {
       // predictor: W on its stencil (value box + 2), one kernel on the cells
       st1_prim.add(q, grow(g.vb1, 2, dims));
@@ -500,7 +600,7 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
     }
     if (fused) st2_upd.add_tiles(q, g.vb2, tz);
     else st2_upd.add(q, g.vb2);
-    if (summed) st2_sum.add_tiles(q, g.vb2, tz, kSumTX, kSumTY);
+    if (summed) add_sum(st2_sum, q, g.vb2);
   }
   // stage 1's lists, then stage 2's (in the order of kPrim .. kSum)
   enum { kPrim, kFlux, kFbc, kUpd, kSum, kStageLists };
@@ -548,6 +648,9 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
     h = fixed->host;
   } else {
     int rc = ensure_arena(c, off);
+    // the face sums take more scratch than the separate kernels
+    if (rc == MFM_ERR_NOMEM && choose && summed)
+      return run_batch(c, Ct, nct, in, n, new_dt, min_cell, level_dt, min_patch, s, fixed, true);
     if (rc) return rc;
     rc = ensure_hbuf(c, host_need);
     if (rc) return rc;
@@ -654,7 +757,8 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
     L.upd = rl(l0 + kUpd);
     L.sum = rl(l0 + kSum);
     L.fused = fused ? 1 : 0;
-    L.summed = summed ? 1 : 0;
+    L.sum_block = sum_block;
+    L.summed = (summed && !(han && st == 0)) ? 1 : 0;  // not the predictor
     return L;
   };
   if (c->timer) c->timer->n = 0;
@@ -663,7 +767,6 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
   auto enqueue = [&](hipStream_t st) -> int {
     auto launch = [&](const StageLists& L, const StepArgs& S) -> hipError_t {
       const DevPatch* tp = (S.stage == 1 && rk2) ? dp2 : dp;
-      const bool f32 = p.precision == MFM_PREC_FP32_FLUX;
       hipError_t e3 = f32 ? launch_stage<float>(C0, ct, tp, L, S, dtp, idp, st, c->timer)
                           : launch_stage<double>(C0, ct, tp, L, S, dtp, idp, st, c->timer);
       if (e3 != hipSuccess) return e3;
@@ -680,23 +783,23 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
     hipError_t e2;
     if (han) {
       // predictorHancock with dt/2, then correctorHancock with dt
-      StepArgs S1{0.5, 0, 0, 0, 0, 0, 0, 0, c->walk_tile, c->walk_xcd, 1, tz};
+      StepArgs S1{0.5, 0, 0, 0, 0, 0, 0, 0, c->walk_tile, c->walk_xcd, 1};
       e2 = launch(stage(0), S1);
       if (e2 != hipSuccess) return hipfail(c, e2, "predictor launch");
       if (c->timer) n_stage1 = c->timer->n;
-      StepArgs S2{1.0, 1, 0, 0, 0, 2, 1, 0, c->walk_tile, c->walk_xcd, 2, tz};
+      StepArgs S2{1.0, 1, 0, 0, 0, 2, 1, 0, c->walk_tile, c->walk_xcd, 2};
       e2 = launch(stage(1), S2);
       if (e2 != hipSuccess) return hipfail(c, e2, "corrector launch");
     } else if (rk2) {
-      StepArgs S1{1.0, 0, 0, 1, 0, 0, 0, 1, c->walk_tile, c->walk_xcd, 0, tz};
+      StepArgs S1{1.0, 0, 0, 1, 0, 0, 0, 1, c->walk_tile, c->walk_xcd, 0};
       e2 = launch(stage(0), S1);
       if (e2 != hipSuccess) return hipfail(c, e2, "stage 1 launch");
       if (c->timer) n_stage1 = c->timer->n;
-      StepArgs S2{0.5, 1, 1, 0, 1, 1, 1, 0, c->walk_tile, c->walk_xcd, 0, tz};
+      StepArgs S2{0.5, 1, 1, 0, 1, 1, 1, 0, c->walk_tile, c->walk_xcd, 0};
       e2 = launch(stage(1), S2);
       if (e2 != hipSuccess) return hipfail(c, e2, "stage 2 launch");
     } else {
-      StepArgs S{1.0, 0, 0, 0, 0, 2, 1, 0, c->walk_tile, c->walk_xcd, 0, tz};
+      StepArgs S{1.0, 0, 0, 0, 0, 2, 1, 0, c->walk_tile, c->walk_xcd, 0};
       e2 = launch(stage(1), S);
       if (e2 != hipSuccess) return hipfail(c, e2, "first-order launch");
     }
@@ -714,7 +817,7 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
                                   (long long)off_ct, (long long)off_dtp, (long long)off_idp,
                                   (long long)off_dto, (long long)off_ido, dims, p.time_approx,
                                   p.precision, C0.nf, C0.dedner, c->walk_tile,
-                                  c->walk_xcd, mode, tz};
+                                  c->walk_xcd, mode, tz, sum_block};
     for (int l = 0; l < kLists; ++l) {
       key.push_back((long long)off_reg[l]);
       key.push_back((long long)lists[l]->v.size());

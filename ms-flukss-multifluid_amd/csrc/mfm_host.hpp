@@ -142,9 +142,11 @@ struct PatchIn {
   double dt, dx, time;
 };
 
+// separate: MFM_STAGE_AUTO takes the separate kernels (too little memory for
+// the face sums' scratch).
 int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
               double* new_dt, int* min_cell, double* level_dt, int* min_patch,
-              hipStream_t s, const FixedScratch* fixed = nullptr);
+              hipStream_t s, const FixedScratch* fixed = nullptr, bool separate = false);
 // Resolves, once per device, the address of the fixed scratch of the
 // allocation-free entry point on the context's device (mfm_noalloc.hip).
 int fixed_scratch_setup(mfm_ctx* c);

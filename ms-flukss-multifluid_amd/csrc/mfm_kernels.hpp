@@ -46,6 +46,7 @@ struct Region {
   int n[3];
   int blk0;
   int dir;
+  int tx, ty, tz;   // tile lists: the column tile and planes of a z-chunk
 };
 
 struct RegionList {
@@ -79,6 +80,7 @@ struct StageLists {
   FaceList flux, fbc;
   int fused;        // upd is a list of k_stage tiles (interior faces and the
                     // update in one launch); flux is then unused
+  int sum_block;    // threads per block of the face-sum kernels
   int summed;       // sum is a list of tiles whose face sums (D) the face-sum
                     // kernels form; k_update then reads D; flux unused
 };
@@ -96,7 +98,6 @@ struct StepArgs {
   int xcd_order;       // work walk: 1 = renumber blocks per XCD
   int hancock;         // 0: Euler / RK2 stage; 1: Hancock predictor;
                        // 2: Hancock corrector
-  int tz;              // k_stage: planes of one z-chunk of a tile
 };
 
 // Optional kernel timing: a pair of events brackets every launch on the
@@ -134,13 +135,14 @@ hipError_t launch_stage_fused(const Consts& C, const Consts* CT, const DevPatch*
                               const StageLists& L, const StepArgs& A, double* dt_part,
                               long* idx_part, hipStream_t s, KernelTimer* T);
 
-// Column tile of the face-sum kernels (k_fsum): long in x, so that the
-// faces a wavefront solves lie along contiguous rows; one thread per column.
-// A tile solves (TX+1)·TY + TX·(TY+1) + TX·TY faces per plane in whole
-// wavefront passes: 14 passes per 256 columns for 64 x 4, 26 per 512 for
-// 64 x 8 (7 % fewer per cell; 11.99 against 12.41 ms per 256^3 step), while
-// 64 x 16 (50 per 1024, one block per CU) is slower again (12.31 ms).
-constexpr int kSumTX = 64, kSumTY = 8, kSumBlock = kSumTX * kSumTY;
+// Tiles of the face-sum kernels: tx x ty columns, at most one per thread of a
+// block of NT threads (256, or 512 in FP32), whose faces of one plane --
+// (tx+1) ty + tx (ty+1) + tx ty -- fit the LDS slots (64 x 8 or 64 x 4 columns,
+// and any shape of no more columns and faces).  FP64 with psi: fewer, for the
+// 64 KB that a block may declare.
+constexpr int sum_slots(int nt, int fsize, int dedner) {
+  return nt == 512 ? 1608 : (fsize == 8 && dedner ? 808 : 836);
+}
 
 // Summed stages: the face-sum kernels over L.sum (after launch_stage has run
 // k_prim and the boundary-face fluxes), then k_update reading their sums.

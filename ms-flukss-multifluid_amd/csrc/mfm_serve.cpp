@@ -79,7 +79,7 @@ size_t request_bytes(const mfm_params& cls, int mode, const Consts& C, const HBo
   if (cls.time_approx == MFM_TIME_HANCOCK) b += align256(cells * C.nc * fs);  // W of U_pred
   if (tiles && mode == MFM_STAGE_FUSED && cls.time_approx == MFM_TIME_RK2)
     b += align256(cells * C.nc * fs);             // W of U*
-  if (tiles && mode == MFM_STAGE_SUMMED && cls.precision == MFM_PREC_FP32_FLUX)
+  if (!cls.char_reconstruction && mode == MFM_STAGE_SUMMED)
     b += align256(cells * (C.nc + 1) * fs);       // face sums
   HBox v1 = cls.time_approx == MFM_TIME_RK2 ? grow(valid, 2, dims)
             : (cls.time_approx == MFM_TIME_HANCOCK ? grow(valid, 1, dims) : valid);
