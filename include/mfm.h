@@ -252,23 +252,26 @@ int mfm_ctx_get_timing(mfm_ctx* ctx, int stage, int kind, double* ms,
  * MFM_STAGE_SEPARATE: per-direction flux kernels writing the face
  * fluxes, then k_update.  MFM_STAGE_SUMMED: after k_prim and the
  * boundary-face kernel, one tile kernel per fluid group (the plasma with
- * psi and the normal B, then each neutral fluid) solves the interior faces
- * of a 64 x 8 column tile, z-chunks of tz planes (default 8), into LDS and
- * writes per cell the face-flux differences summed over the directions;
- * k_update applies those sums (FP32-flux build only; the FP64 build keeps
- * the reference's order, the directions one at a time, and runs the
- * separate kernels in this mode).  MFM_STAGE_FUSED: one tile kernel per stage
- * solves every face and updates the cells; the face fluxes never reach HBM,
- * but its register budget makes it slower on the 256^3 workload.
- * MFM_STAGE_AUTO (default): per batch, the summed stages in the FP32-flux
- * build when the batch's cells fill at least 3/4 of their 64 x 8 column
- * tiles (12.0 against 13.9-14.2 ms per step on the 256^3 workload), else the
- * separate kernels; the allocation-free entry point always takes the
- * separate kernels.  AUTO decides per call: in the FP32-flux build a patch
- * updated alone and in a level can then take different structures (results
- * equal within the FP32 bar, not bit for bit); a fixed mode gives the same
- * bits whatever the batch.  The Hancock scheme and characteristic slopes
- * always use the separate kernels.                                         */
+ * psi and the normal B, the neutral fluids) solves the interior faces of a
+ * column tile, z-chunks of tz planes (default 8), into LDS and writes per cell
+ * the face-flux differences summed over the directions, or in the FP64 build
+ * the state with the directions applied one after the other (the separate
+ * kernels' bits); k_update finishes the stage from those.  The Hancock
+ * corrector takes it too.  MFM_STAGE_FUSED: one tile kernel per stage solves
+ * every face and updates the cells; the face fluxes never reach HBM, but its
+ * register budget makes it slower on the 256^3 workload (the Hancock scheme
+ * runs the separate kernels in this mode).
+ * MFM_STAGE_AUTO (default): per call, the summed stages where they are the
+ * faster ones -- in the FP32-flux build when the cells fill at least 3/4 of
+ * their 64 x 8 column tiles (12.2 against 13.9-14.2 ms per step on the 256^3
+ * workload), and in either build from a number of cells on that depends on
+ * the fluids and the scheme, with shorter z-chunks (tz at most) for small
+ * calls -- else the separate kernels; the allocation-free entry point always
+ * takes the separate kernels.  AUTO decides per call: in the FP32-flux build
+ * a patch updated alone and in a level can then take different structures
+ * (results equal within the FP32 bar, not bit for bit; the FP64 build gives
+ * the same bits in both); a fixed mode gives the same bits whatever the
+ * batch.  Characteristic slopes always use the separate kernels.            */
 enum { MFM_STAGE_SEPARATE = 0, MFM_STAGE_FUSED = 1, MFM_STAGE_SUMMED = 2, MFM_STAGE_AUTO = 3 };
 int mfm_ctx_set_stage_kernel(mfm_ctx* ctx, int mode, int tz);
 

@@ -144,7 +144,8 @@ struct RegionBuilder {
 // faces of one direction take whole wavefronts (issue) in whole rounds of the
 // block's threads (a barrier waits for the last): the shape with the smallest
 // sum of both over the box, the wider one on a tie.
-// TILE_MEASURED
+// (Against the fewest wavefronts alone, 64 x 8 at 256^3: 32 x 15 takes 24.40 instead
+// of 24.51 ms per two steps; a level of 8^3 .. 32^3 boxes 4.61 instead of 4.79 ms.)
 struct Tile { int tx, ty; };
 long tile_rounds(const Tile& t, int block) {
   auto rounds = [&](long f) { return (f + block - 1) / block; };

@@ -35,12 +35,12 @@ struct mfm_ctx {
   // work walk of the region kernels (row tile in (y, z), XCD renumbering)
   int walk_tile = 8;
   int walk_xcd = 1;
-  // kernel structure of RK2 / first-order stages (MFM_STAGE_*): separate
-  // per-direction flux kernels, the fused stage kernel (k_stage), the
-  // face-sum tile kernels (k_fsum) before k_update, or the choice per batch
-  // between separate and summed (AUTO); the tile kernels walk z-chunks of
-  // stage_tz planes per block (8: 12.01 / 11.75 against 12.03 / 12.07 ms per
-  // 256^3 step for 16, 12.26 for 12, 12.10 for 4, 12.56 for 32)
+  // kernel structure of a stage (MFM_STAGE_*): separate flux kernels, the
+  // fused stage kernel (k_stage), the face-sum tile kernels before k_update,
+  // or the choice per call between separate and summed (AUTO); the tile
+  // kernels walk z-chunks of at most stage_tz planes per block (8: 12.01 /
+  // 11.75 against 12.03 / 12.07 ms per 256^3 step for 16, 12.26 for 12, 12.10
+  // for 4, 12.56 for 32; small calls take fewer, kAutoBlocks)
   int stage_mode = MFM_STAGE_AUTO;
   int stage_tz = 8;
   // host staging of the allocation-free entry point (tables and results of
