@@ -61,19 +61,18 @@ __device__ __forceinline__ void copy_cell(double* dp, long dcs, const double* sp
     if (q < m) dp[(c0 + q) * dcs] = v[q];
 }
 
-__global__ __launch_bounds__(kFB) void k_rect_copy(
-    const CopyRect* __restrict__ R, int nr, const FillFab* __restrict__ Sn,
+// One wavefront per block: a corner of a ghost layer 4 deep is 64 cells, and
+// the rectangle of a block comes from a table instead of a search through them
+// all: 365 -> 338 us for 343 boxes of 16^3 (4 ghosts, 23 components, 2.9 TB/s of
+// the cells' bytes; rows of 4 cells touch whole cache lines).
+__global__ __launch_bounds__(kRectBlock) void k_rect_copy(
+    const CopyRect* __restrict__ R, const int* __restrict__ of, const FillFab* __restrict__ Sn,
     const FillFab* __restrict__ So, const FillFab* __restrict__ D, int nc,
     double a, double b, int mode) {
   const int bx = xcd_block();
-  int lo = 0, hi = nr - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (R[mid].blk0 <= bx) lo = mid; else hi = mid - 1;
-  }
-  const CopyRect r = R[lo];
+  const CopyRect r = R[of[bx]];
   // (2^32 cells of one component would be 34 GB)
-  const unsigned t = (unsigned)(bx - r.blk0) * kFB + threadIdx.x;
+  const unsigned t = (unsigned)(bx - r.blk0) * kRectBlock + threadIdx.x;
   const unsigned n01 = (unsigned)r.n[0] * r.n[1];
   if (t >= n01 * r.n[2]) return;
   const int k = (int)(t / n01);
@@ -287,12 +286,12 @@ __global__ __launch_bounds__(kFB) void k_fill_interp(InterpArgs A) {
 unsigned comp_blocks(int nc, int per) { return (unsigned)((nc + per - 1) / per); }
 }  // namespace
 
-hipError_t launch_rect_copy(const CopyRect* R, int nr, int nblk,
+hipError_t launch_rect_copy(const CopyRect* R, const int* of, int nblk,
                             const FillFab* src_new, const FillFab* src_old,
                             const FillFab* dst, int nc, double a, double b,
                             int mode, hipStream_t s) {
-  if (nr <= 0 || nblk <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_rect_copy, dim3((unsigned)nblk, comp_blocks(nc, kCopyComps)), dim3(kFB), 0, s, R, nr,
+  if (nblk <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_rect_copy, dim3((unsigned)nblk, comp_blocks(nc, kCopyComps)), dim3(kRectBlock), 0, s, R, of,
                      src_new, src_old, dst, nc, a, b, mode);
   return hipGetLastError();
 }

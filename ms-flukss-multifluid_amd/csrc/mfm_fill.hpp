@@ -54,7 +54,9 @@ struct InterpArgs {
   double c_centre, c_side, dxc, dxf, coeff, tiny;
 };
 
-hipError_t launch_rect_copy(const CopyRect* R, int nr, int nblk,
+// Blocks of the rectangle copies: of: each block's rectangle.
+constexpr int kRectBlock = 64;
+hipError_t launch_rect_copy(const CopyRect* R, const int* of, int nblk,
                             const FillFab* src_new, const FillFab* src_old,
                             const FillFab* dst, int nc, double a, double b,
                             int mode, hipStream_t s);

@@ -40,6 +40,7 @@ using mfm::host::grow;
 namespace {
 
 constexpr int kFB = 256;
+using mfm::kRectBlock;
 
 int fdiv(int a, int r) { return a >= 0 ? a / r : -((-a - 1) / r) - 1; }
 
@@ -202,6 +203,7 @@ struct mfm_fill_plan {
   std::string err;
   std::vector<HBox> fine, crse;
   std::vector<CopyRect> xr;      // exchange
+  std::vector<int> xb;           // the exchange rectangle of each block
   int xr_blk = 0;
   std::vector<GatherCell> gc;    // gather
   std::vector<int2> cells;
@@ -214,6 +216,7 @@ struct mfm_fill_plan {
   char* dmem = nullptr;
   size_t dbytes = 0;
   CopyRect* d_xr = nullptr;
+  int* d_xb = nullptr;
   GatherCell* d_gc = nullptr;
   int2* d_cells = nullptr;
   uint8_t* d_flags = nullptr;
@@ -257,7 +260,7 @@ void add_rect(std::vector<CopyRect>& v, int& nblk, int src, int dst,
     r.n[d] = (int)dstbox.n(d);
   }
   r.blk0 = nblk;
-  nblk += (int)((cells + kFB - 1) / kFB);
+  nblk += (int)((cells + kRectBlock - 1) / kRectBlock);
   v.push_back(r);
 }
 
@@ -302,6 +305,7 @@ int build(mfm_fill_plan* P, const mfm_params* p, const mfm_box* boxes, int n,
         HBox I = inter(G, shift(P->fine[j], s.data()));
         if (empty(I)) continue;
         add_rect(P->xr, P->xr_blk, j, i, I, s.data());
+        P->xb.resize((size_t)P->xr_blk, (int)P->xr.size() - 1);
         P->x_cells += I.size();
       }
     }
@@ -491,19 +495,21 @@ int upload(mfm_ctx* c, mfm_fill_plan* P) {
   }
   using mfm::host::align256;
   const size_t b_xr = align256(P->xr.size() * sizeof(CopyRect));
+  const size_t b_xb = align256(P->xb.size() * sizeof(int));
   const size_t b_gc = align256(P->gc.size() * sizeof(GatherCell));
   const size_t b_cells = align256(P->cells.size() * sizeof(int2));
   const size_t b_flags = align256(P->flags.size());
   const size_t b_fp = align256(P->fp.size() * sizeof(FillPatch));
   const size_t b_wfab = align256(P->fp.size() * sizeof(FillFab));
   const size_t b_work = align256(P->work_doubles * sizeof(double));
-  const size_t total = b_xr + b_gc + b_cells + b_flags + b_fp + b_wfab + b_work + 256;
+  const size_t total = b_xr + b_xb + b_gc + b_cells + b_flags + b_fp + b_wfab + b_work + 256;
   e = hipMalloc((void**)&P->dmem, total);
   if (e != hipSuccess) { P->dmem = nullptr; return mfm::host::fail(c, MFM_ERR_NOMEM, "hipMalloc of the fill plan failed"); }
   P->device = dev;
   P->dbytes = total;
   char* q = P->dmem;
   P->d_xr = (CopyRect*)q; q += b_xr;
+  P->d_xb = (int*)q; q += b_xb;
   P->d_gc = (GatherCell*)q; q += b_gc;
   P->d_cells = (int2*)q; q += b_cells;
   P->d_flags = (uint8_t*)q; q += b_flags;
@@ -519,6 +525,7 @@ int upload(mfm_ctx* c, mfm_fill_plan* P) {
   }
   struct Up { void* dst; const void* src; size_t bytes; } ups[] = {
       {P->d_xr, P->xr.data(), P->xr.size() * sizeof(CopyRect)},
+      {P->d_xb, P->xb.data(), P->xb.size() * sizeof(int)},
       {P->d_gc, P->gc.data(), P->gc.size() * sizeof(GatherCell)},
       {P->d_cells, P->cells.data(), P->cells.size() * sizeof(int2)},
       {P->d_flags, P->flags.data(), P->flags.size()},
@@ -638,7 +645,7 @@ int mfm_fill_plan_info(const mfm_fill_plan* P, long* xc, long* fc, long* cc,
   if (cc) *cc = (long)P->cells.size();
   if (bytes) {
     using mfm::host::align256;
-    *bytes = align256(P->xr.size() * sizeof(CopyRect)) + align256(P->gc.size() * sizeof(GatherCell)) +
+    *bytes = align256(P->xr.size() * sizeof(CopyRect)) + align256(P->xb.size() * sizeof(int)) + align256(P->gc.size() * sizeof(GatherCell)) +
              align256(P->cells.size() * sizeof(int2)) + align256(P->flags.size()) +
              align256(P->fp.size() * sizeof(FillPatch)) + align256(P->fp.size() * sizeof(FillFab)) +
              align256(P->work_doubles * sizeof(double)) + 256;
@@ -658,7 +665,7 @@ int mfm_level_exchange_dev(mfm_ctx* c, mfm_fill_plan* P, const mfm_fab* U,
   rc = stage_tables(c, P, 0, U, nullptr, nullptr, s);
   if (rc) return rc;
   const FillFab* T = P->tab[0].d;
-  hipError_t e = mfm::launch_rect_copy(P->d_xr, (int)P->xr.size(), P->xr_blk, T, T, T, P->nc,
+  hipError_t e = mfm::launch_rect_copy(P->d_xr, P->d_xb, P->xr_blk, T, T, T, P->nc,
                                        1.0, 0.0, 0, s);
   if (e != hipSuccess) return mfm::host::hipfail(c, e, "exchange launch");
   return MFM_OK;

@@ -172,30 +172,44 @@ __global__ __launch_bounds__(kB) void k_init(Consts C, double* U, Geo G,
 }
 
 // Periodic images of a one-box level: every ghost cell copies the valid
-// cell congruent to it modulo the box size.
+// cell congruent to it modulo the box size.  blockIdx.y: a chunk of the
+// components, whose loads leave before its stores (the compiler may not move
+// a load of U across a store to it: one component at a time took a memory
+// latency each: 5.7 -> 4.7 us for 8 components of an 800-cell tube).
+constexpr int kPeriodicComps = 8;
 __global__ __launch_bounds__(kB) void k_fill_periodic(double* U, Geo G, int nc,
                                                       int vlo0, int vlo1,
                                                       int vlo2, int vn0,
                                                       int vn1, int vn2,
                                                       int dims) {
-  int a, b, c;
-  const long t = (long)blockIdx.x * kB + threadIdx.x;
-  if (!unravel(t, G.un, a, b, c)) return;
-  int idx[3] = {G.ulo[0] + a, G.ulo[1] + b, G.ulo[2] + c};
+  // (the host rejects FABs of 2^31 cells or more)
+  const unsigned t = blockIdx.x * kB + threadIdx.x;
+  const unsigned n0 = (unsigned)G.un[0], n1 = (unsigned)G.un[1];
+  const unsigned row = t / n0, c = row / n1;
+  if (c >= (unsigned)G.un[2]) return;
+  const int idx[3] = {G.ulo[0] + (int)(t - row * n0), G.ulo[1] + (int)(row - c * n1),
+                      G.ulo[2] + (int)c};
   const int vlo[3] = {vlo0, vlo1, vlo2}, vn[3] = {vn0, vn1, vn2};
   int src[3] = {idx[0], idx[1], idx[2]};
   bool ghost = false;
   for (int d = 0; d < dims; ++d) {
     int o = idx[d] - vlo[d];
+    if (o >= 0 && o < vn[d]) continue;
     o = ((o % vn[d]) + vn[d]) % vn[d];
     src[d] = vlo[d] + o;
-    if (src[d] != idx[d]) ghost = true;
+    ghost = true;
   }
   if (!ghost) return;
-  const long dst = t;
   const long s = (long)(src[0] - G.ulo[0]) +
                  (long)G.un[0] * ((long)(src[1] - G.ulo[1]) + (long)G.un[1] * (src[2] - G.ulo[2]));
-  for (int q = 0; q < nc; ++q) U[dst + q * G.ucs] = U[s + q * G.ucs];
+  const int c0 = (int)blockIdx.y * kPeriodicComps;
+  double v[kPeriodicComps];
+#pragma unroll
+  for (int q = 0; q < kPeriodicComps; ++q)
+    if (c0 + q < nc) v[q] = U[s + (c0 + q) * G.ucs];
+#pragma unroll
+  for (int q = 0; q < kPeriodicComps; ++q)
+    if (c0 + q < nc) U[t + (c0 + q) * G.ucs] = v[q];
 }
 }  // namespace
 
@@ -219,7 +233,9 @@ hipError_t launch_fill_periodic(double* U, const int ulo[3], const int un[3],
   for (int d = 0; d < 3; ++d) { G.ulo[d] = ulo[d]; G.un[d] = un[d]; G.lo[d] = 0; G.n[d] = 0; }
   G.ucs = ucs;
   const long tot = (long)un[0] * un[1] * un[2];
-  hipLaunchKernelGGL(k_fill_periodic, dim3((unsigned)((tot + kB - 1) / kB)),
+  hipLaunchKernelGGL(k_fill_periodic,
+                     dim3((unsigned)((tot + kB - 1) / kB),
+                          (unsigned)((nc + kPeriodicComps - 1) / kPeriodicComps)),
                      dim3(kB), 0, s, U, G, nc, vlo[0], vlo[1], vlo[2], vn[0],
                      vn[1], vn[2], dims);
   return hipGetLastError();
