@@ -850,8 +850,9 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
   }
   double* hdt = reinterpret_cast<double*>(h + table_bytes);
   long* hid = reinterpret_cast<long*>(h + table_bytes + align256(sizeof(double) * n));
-  e = hipMemcpyAsync(hdt, A + off_dto, sizeof(double) * n, hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(hid, A + off_ido, sizeof(long) * n, hipMemcpyDeviceToHost, s);
+  // the cell indices follow the time steps at the same distance on both sides
+  e = hipMemcpyAsync(hdt, A + off_dto, (off_ido - off_dto) + sizeof(long) * n,
+                     hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return hipfail(c, e, "patch update");
   if (c->timer) {
@@ -942,8 +943,8 @@ int run_dt(mfm_ctx* c, const Consts& C0, const mfm_fab& U, const mfm_box& box,
                         reinterpret_cast<double*>(A + off_dto), reinterpret_cast<long*>(A + off_ido), s);
   double* hdt = reinterpret_cast<double*>(c->hbuf + off_c + align256(sizeof(Consts)));
   long* hid = reinterpret_cast<long*>(c->hbuf + off_c + align256(sizeof(Consts)) + 256);
-  if (e == hipSuccess) e = hipMemcpyAsync(hdt, A + off_dto, sizeof(double), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(hid, A + off_ido, sizeof(long), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(hdt, A + off_dto, (off_ido - off_dto) + sizeof(long), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return hipfail(c, e, "compute_dt");
   double d = *hdt;

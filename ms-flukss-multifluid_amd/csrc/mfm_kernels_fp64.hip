@@ -15,8 +15,13 @@ template hipError_t launch_update_summed<double>(const Consts&, const Consts*, c
 hipError_t launch_dt_final(const RegionList& L, const double* dt_part,
                            const long* idx_part, double* dt_out, long* idx_out,
                            hipStream_t s) {
-  hipLaunchKernelGGL(k_dt_final, dim3(L.n), dim3(kBlock), 0, s, L.r, L.n,
-                     L.nblk, dt_part, idx_part, dt_out, idx_out);
+  // one patch with many partials: a block of 1024 threads per region
+  if (L.nblk > 1024 * L.n)
+    hipLaunchKernelGGL((k_dt_final<1024>), dim3(L.n), dim3(1024), 0, s, L.r, L.n,
+                       L.nblk, dt_part, idx_part, dt_out, idx_out);
+  else
+    hipLaunchKernelGGL((k_dt_final<kBlock>), dim3(L.n), dim3(kBlock), 0, s, L.r, L.n,
+                       L.nblk, dt_part, idx_part, dt_out, idx_out);
   return hipGetLastError();
 }
 hipError_t launch_dt_only(const Consts& C, const Consts* CT, const DevPatch* P,
