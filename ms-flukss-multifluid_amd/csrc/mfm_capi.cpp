@@ -197,6 +197,13 @@ struct TileCache {
   }
 };
 
+// Whether every physical ghost state of the problem is a constant (RIEMANNGS;
+// HELIOGS's plasma and first neutral population): W keeps it from one RK2
+// stage to the next.
+bool fixed_ghosts(const Consts& C) {
+  return C.problem == MFM_PROBLEM_RIEMANN || (C.problem == MFM_PROBLEM_HELIO && C.nf <= 2);
+}
+
 // A face list under construction: the regions direction by direction, and
 // where each direction ends.
 struct FaceBuilder : RegionBuilder {
@@ -578,6 +585,8 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
           rest.hi[d] = g.vb1.hi[d];
         }
       }
+    } else if (rk2 && !fused && fixed_ghosts(Ct[pin[q].cidx])) {
+      // the first stage leaves W of U* on vb1 and its ghost states hold
     } else if (rk2) {
       // the first stage leaves W of U* on vb1; the second stage only needs
       // the physical ghost cells of grow(vb2, 2) outside it
@@ -784,23 +793,23 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
     hipError_t e2;
     if (han) {
       // predictorHancock with dt/2, then correctorHancock with dt
-      StepArgs S1{0.5, 0, 0, 0, 0, 0, 0, 0, c->walk_tile, c->walk_xcd, 1};
+      StepArgs S1{0.5, 0, 0, 0, 0, 0, 0, 0, c->walk_tile, c->walk_xcd, 1, 0};
       e2 = launch(stage(0), S1);
       if (e2 != hipSuccess) return hipfail(c, e2, "predictor launch");
       if (c->timer) n_stage1 = c->timer->n;
-      StepArgs S2{1.0, 1, 0, 0, 0, 2, 1, 0, c->walk_tile, c->walk_xcd, 2};
+      StepArgs S2{1.0, 1, 0, 0, 0, 2, 1, 0, c->walk_tile, c->walk_xcd, 2, 0};
       e2 = launch(stage(1), S2);
       if (e2 != hipSuccess) return hipfail(c, e2, "corrector launch");
     } else if (rk2) {
-      StepArgs S1{1.0, 0, 0, 1, 0, 0, 0, 1, c->walk_tile, c->walk_xcd, 0};
+      StepArgs S1{1.0, 0, 0, 1, 0, 0, 0, 1, c->walk_tile, c->walk_xcd, 0, 0};
       e2 = launch(stage(0), S1);
       if (e2 != hipSuccess) return hipfail(c, e2, "stage 1 launch");
       if (c->timer) n_stage1 = c->timer->n;
-      StepArgs S2{0.5, 1, 1, 0, 1, 1, 1, 0, c->walk_tile, c->walk_xcd, 0};
+      StepArgs S2{0.5, 1, 1, 0, 1, 1, 1, 0, c->walk_tile, c->walk_xcd, 0, fused ? 0 : 1};
       e2 = launch(stage(1), S2);
       if (e2 != hipSuccess) return hipfail(c, e2, "stage 2 launch");
     } else {
-      StepArgs S{1.0, 0, 0, 0, 0, 2, 1, 0, c->walk_tile, c->walk_xcd, 0};
+      StepArgs S{1.0, 0, 0, 0, 0, 2, 1, 0, c->walk_tile, c->walk_xcd, 0, 0};
       e2 = launch(stage(1), S);
       if (e2 != hipSuccess) return hipfail(c, e2, "first-order launch");
     }

@@ -540,6 +540,17 @@ __device__ __forceinline__ void char_synthesis(const CharBasis<T>& B, const T* a
 // ---------------------------------------------------- cons -> prim (FP64) --
 // CONSTOPRIM / CONSTOPRIM_MF (srcIdeal/PatchIdealMHDF.ChF:143-189,
 // srcIdeal/PatchMHDMFF.ChF:5-80): the multi-fluid version floors rho.
+// One neutral fluid (5 components).
+__device__ __forceinline__ void neutral_to_prim(const Consts& C, const double* u, double* w) {
+  const double r = fmaxr(C.smallr, u[0]);
+  const double jr = 1.0 / r;
+  const double ax = u[1] * jr, ay = u[2] * jr, az = u[3] * jr;
+  const double k2 = u[1] * ax + u[2] * ay + u[3] * az;
+  double q = C.hgamma * (u[4] - 0.5 * k2);
+  q = fmaxr(C.smallp, q);
+  w[0] = r; w[1] = ax; w[2] = ay; w[3] = az; w[4] = q;
+}
+
 template <class S>
 __device__ __forceinline__ void cons_to_prim(const Consts& C, const double* u,
                                              double* w) {
@@ -555,16 +566,8 @@ __device__ __forceinline__ void cons_to_prim(const Consts& C, const double* u,
   w[5] = u[5]; w[6] = u[6]; w[7] = u[7];
   if (S::DED) w[8] = u[8];
 #pragma unroll
-  for (int f = 1; f < S::NF; ++f) {
-    const int s = S::IRN + 5 * (f - 1);
-    const double r = fmaxr(C.smallr, u[s]);
-    const double jr = 1.0 / r;
-    const double ax = u[s + 1] * jr, ay = u[s + 2] * jr, az = u[s + 3] * jr;
-    const double k2 = u[s + 1] * ax + u[s + 2] * ay + u[s + 3] * az;
-    double q = C.hgamma * (u[s + 4] - 0.5 * k2);
-    q = fmaxr(C.smallp, q);
-    w[s] = r; w[s + 1] = ax; w[s + 2] = ay; w[s + 3] = az; w[s + 4] = q;
-  }
+  for (int f = 1; f < S::NF; ++f)
+    neutral_to_prim(C, u + S::IRN + 5 * (f - 1), w + S::IRN + 5 * (f - 1));
 }
 
 // ---------------------------------------------------------- MHD fluxes --

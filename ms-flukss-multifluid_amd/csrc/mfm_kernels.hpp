@@ -98,6 +98,8 @@ struct StepArgs {
   int xcd_order;       // work walk: 1 = renumber blocks per XCD
   int hancock;         // 0: Euler / RK2 stage; 1: Hancock predictor;
                        // 2: Hancock corrector
+  int ghosts_set;      // k_prim: W holds the problem's constant ghost states
+                       // from the first RK2 stage
 };
 
 // Optional kernel timing: a pair of events brackets every launch on the
