@@ -23,7 +23,8 @@ def test_dt_of_many_blocks(oracle_mod, n, uniform):
         U[:] = U[:, 5:6, 5:6, 5:6]
     vhi = tuple(v - 1 for v in n)
     ctx = mfmhd.Context(p)
-    dt, cell = ctx.compute_dt(GpuPatch(U, lo).fab, mfmhd.Box.of((0, 0, 0), vhi), 0.05)
+    g = GpuPatch(U, lo)  # holds the device memory during the call
+    dt, cell = ctx.compute_dt(g.fab, mfmhd.Box.of((0, 0, 0), vhi), 0.05)
     want, wcell = oracle_mod.compute_dt(p, U, lo, (0, 0, 0), vhi, 0.05)
     assert abs(dt - want) <= 1e-14 * want
     assert tuple(cell) == ((0, 0, 0) if uniform else tuple(wcell))
