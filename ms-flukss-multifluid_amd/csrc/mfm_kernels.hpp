@@ -46,7 +46,8 @@ struct Region {
   int n[3];
   int blk0;
   int dir;
-  int tx, ty, tz;   // tile lists: the column tile and planes of a z-chunk
+  int tx, ty, tz;   // tile lists: the column tile and planes of a z-chunk;
+                    // walked face lists: tz faces per thread
 };
 
 struct RegionList {
@@ -75,11 +76,13 @@ struct FaceBlocks {
 // flux: interior faces; fbc: faces on a physical (non-periodic) domain
 // boundary (in blocks of kBcBlock).
 constexpr int kBcBlock = 64;
+constexpr int kCharLanes = 63;  // faces of a row per wavefront of k_flux_plasma_char
 struct StageLists {
   RegionList prim, upd, sum;
   FaceList flux, fbc;
   int fused;        // upd is a list of k_stage tiles (interior faces and the
                     // update in one launch); flux is then unused
+  int char_walk;    // flux is the list of k_flux_plasma_char
   int sum_block;    // threads per block of the face-sum kernels
   int summed;       // sum is a list of tiles whose face sums (D) the face-sum
                     // kernels form; k_update then reads D; flux unused
