@@ -42,6 +42,7 @@ UNITS = [
     ("mfm_init.hip", ["-ffp-contract=off"]),
     ("mfm_capi.cpp", ["-ffp-contract=off"]),
     ("mfm_serve.cpp", ["-ffp-contract=off"]),
+    ("mfm_hostcopy.cpp", []),
     ("mfm_fill.hip", ["-ffp-contract=off"]),
     ("mfm_sync.hip", ["-ffp-contract=off"]),
     ("mfm_fill_plan.cpp", ["-ffp-contract=off"]),

@@ -64,6 +64,14 @@ int ensure_arena(mfm_ctx* c, size_t bytes) {
   }
   size_t want = bytes + bytes / 8;
   hipError_t e = hipMalloc((void**)&c->arena, want);
+  if (e != hipSuccess && c->host_u && !c->host_busy) {
+    // U's place of the host-buffer entry point is in no call's use now
+    (void)hipGetLastError();
+    (void)hipFree(c->host_u);
+    c->host_u = nullptr;
+    c->host_u_bytes = 0;
+    e = hipMalloc((void**)&c->arena, want);
+  }
   if (e != hipSuccess) {
     c->arena = nullptr;
     (void)hipGetLastError();  // a later launch check must not find this error
@@ -119,14 +127,6 @@ struct RegionBuilder {
     nblk += (int)((cells + blk - 1) / blk);
     v.push_back(r);
   }
-  // a region of a tile kernel: one block per tx x ty column tile and
-  // z-chunk of tz planes
-  void add_tiles(int patch, const HBox& b, int tz, int tx = 16, int ty = 16) {
-    long cells = b.size();
-    if (cells <= 0) return;
-    items += cells;
-    Region r;
-    r.patch = patch;
   // faces of direction dir for k_flux_plasma_char, `walk` per thread in y and z
   void add_walk(int patch, const HBox& b, int dir, int walk) {
     const int at = v.size(), blk0 = nblk;
@@ -139,6 +139,14 @@ struct RegionBuilder {
                                 : n[0] * n[3 - dir] * ((n[dir] + walk - 1) / walk);
     nblk = blk0 + (int)((items + kBlk - 1) / kBlk);
   }
+  // a region of a tile kernel: one block per tx x ty column tile and
+  // z-chunk of tz planes
+  void add_tiles(int patch, const HBox& b, int tz, int tx = 16, int ty = 16) {
+    long cells = b.size();
+    if (cells <= 0) return;
+    items += cells;
+    Region r;
+    r.patch = patch;
     r.dir = 0;
     r.tx = tx;
     r.ty = ty;
@@ -535,14 +543,6 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
   const PatchIn* pin = in;
   RegionBuilder st1_prim, st1_upd, st2_prim, st2_upd, st1_sum, st2_sum;
   FaceBuilder st1_flux, st1_fbc, st2_flux, st2_fbc;
-  auto add_faces = [&](RegionBuilder& in, RegionBuilder& bc, int q, HBox f, int d) {
-    const Consts& Cq = Ct[pin[q].cidx];
-    if (Cq.phys[d]) {
-      if (f.lo[d] == Cq.dom_lo[d]) {
-        HBox b = f;
-        b.hi[d] = b.lo[d];
-        bc.add(q, b, kBcBlock, d);
-        f.lo[d] += 1;
   // Characteristic slopes with one fluid: faces walked per thread, where the
   // threads still fill the chip.  A Hancock step with 1 / 4 / 8 faces per
   // thread: 262k cells 195 / 203 / 216 us, 614k 379 / 377 / 376, 960k 596 / 570 / 583,
@@ -553,6 +553,14 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
     for (int q = 0; q < n; ++q) cells += (double)G[q].vb2.size();
     walk = cells >= 4.0e6 ? 8 : (cells >= 8.0e5 ? 4 : 0);
   }
+  auto add_faces = [&](RegionBuilder& in, RegionBuilder& bc, int q, HBox f, int d) {
+    const Consts& Cq = Ct[pin[q].cidx];
+    if (Cq.phys[d]) {
+      if (f.lo[d] == Cq.dom_lo[d]) {
+        HBox b = f;
+        b.hi[d] = b.lo[d];
+        bc.add(q, b, kBcBlock, d);
+        f.lo[d] += 1;
       }
       if (f.hi[d] == Cq.dom_hi[d] + 1 && f.hi[d] >= f.lo[d]) {
         HBox b = f;
@@ -791,6 +799,7 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
     L.upd = rl(l0 + kUpd);
     L.sum = rl(l0 + kSum);
     L.fused = fused ? 1 : 0;
+    L.char_walk = walk > 0 ? 1 : 0;
     L.sum_block = sum_block;
     L.summed = (summed && !(han && st == 0)) ? 1 : 0;  // not the predictor
     return L;
@@ -799,7 +808,6 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
   int n_stage1 = 0;
   // the whole launch sequence of one update (both stages, dt reduction)
   auto enqueue = [&](hipStream_t st) -> int {
-    L.char_walk = walk > 0 ? 1 : 0;
     auto launch = [&](const StageLists& L, const StepArgs& S) -> hipError_t {
       const DevPatch* tp = (S.stage == 1 && rk2) ? dp2 : dp;
       hipError_t e3 = f32 ? launch_stage<float>(C0, ct, tp, L, S, dtp, idp, st, c->timer)
@@ -1364,6 +1372,7 @@ int mfm_ctx_destroy(mfm_ctx* c) {
   if (c->cap_stream) (void)hipStreamDestroy(c->cap_stream);
   if (c->arena) (void)hipFree(c->arena);
   if (c->hbuf) (void)hipHostFree(c->hbuf);
+  if (c->host_u) (void)hipFree(c->host_u);
   delete c;
   return MFM_OK;
 }
@@ -1447,15 +1456,28 @@ int mfm_patch_update_host(mfm_ctx* c, mfm_fab U, mfm_box valid, double dt,
   if (divB && (!divB->data || divB->ncomp <= 0 || hb(divB->box).size() == 0))
     return fail(c, MFM_ERR_SHAPE, "divB: empty FAB");
   size_t ub_bytes = (size_t)ub.size() * U.ncomp * sizeof(double);
-  double* dU = nullptr;
   std::vector<double*> dF(3, nullptr);
   double* dD = nullptr;
   mfm_fab Fd[3];
   mfm_fab Dd;
   int rc = MFM_OK;
-  hipError_t e = hipMalloc((void**)&dU, ub_bytes);
-  if (e != hipSuccess) return fail(c, MFM_ERR_NOMEM, "hipMalloc(U)");
-  e = hipMemcpy(dU, U.data, ub_bytes, hipMemcpyHostToDevice);
+  hipError_t e = hipSuccess;
+  // U's place on the device stays with the context between calls
+  if (c->host_u_bytes < ub_bytes) {
+    if (c->host_u) (void)hipFree(c->host_u);
+    c->host_u = nullptr;
+    c->host_u_bytes = 0;
+    e = hipMalloc((void**)&c->host_u, ub_bytes);
+    if (e != hipSuccess) {
+      c->host_u = nullptr;
+      (void)hipGetLastError();
+      return fail(c, MFM_ERR_NOMEM, "hipMalloc(U)");
+    }
+    c->host_u_bytes = ub_bytes;
+  }
+  double* dU = c->host_u;
+  const CopySeg whole{0, ub_bytes};
+  e = host_copy(c->link, dU, U.data, &whole, 1, true);
   if (F) {
     for (int d = 0; d < dims && e == hipSuccess; ++d) {
       size_t b = (size_t)hb(F[d].box).size() * F[d].ncomp * sizeof(double);
@@ -1478,11 +1500,22 @@ int mfm_patch_update_host(mfm_ctx* c, mfm_fab U, mfm_box valid, double dt,
   if (!rc) {
     mfm_fab Ud = U;
     Ud.data = dU;
+    c->host_busy = true;
     rc = mfm_patch_update_dev(c, Ud, valid, dt, dx, time, F ? Fd : nullptr,
                               divB ? &Dd : nullptr, new_dt, min_cell, nullptr);
+    c->host_busy = false;
   }
   if (!rc || rc == MFM_ERR_NUMERIC) {
-    e = hipMemcpy(U.data, dU, ub_bytes, hipMemcpyDeviceToHost);
+    // the update writes the valid box only: of each component, the planes
+    // that hold it come back
+    const HBox v = hb(valid);
+    const int top = dims - 1;
+    const size_t plane = (size_t)ub.size() / (size_t)ub.n(top) * sizeof(double);
+    std::vector<CopySeg> seg((size_t)U.ncomp);
+    for (int q = 0; q < U.ncomp; ++q)
+      seg[q] = {((size_t)q * ub.n(top) + (size_t)(v.lo[top] - ub.lo[top])) * plane,
+                (size_t)v.n(top) * plane};
+    e = host_copy(c->link, dU, U.data, seg.data(), U.ncomp, false);
     for (int d = 0; F && d < dims && e == hipSuccess; ++d)
       e = hipMemcpy(F[d].data, dF[d], (size_t)hb(F[d].box).size() * F[d].ncomp * sizeof(double),
                     hipMemcpyDeviceToHost);
@@ -1491,7 +1524,6 @@ int mfm_patch_update_host(mfm_ctx* c, mfm_fab U, mfm_box valid, double dt,
                     hipMemcpyDeviceToHost);
     if (e != hipSuccess) rc = hipfail(c, e, "copy back");
   }
-  (void)hipFree(dU);
   for (int d = 0; d < 3; ++d)
     if (dF[d]) (void)hipFree(dF[d]);
   if (dD) (void)hipFree(dD);

@@ -3,12 +3,25 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "../../include/mfm.h"
 #include "mfm_device.hpp"
 #include "mfm_kernels.hpp"
+
+namespace mfm {
+namespace host {
+struct HostCopier;
+// A context's pinned copy pipeline (mfm_hostcopy.cpp), made by its first large copy.
+struct HostLink {
+  std::mutex mu;
+  HostCopier* copier = nullptr;
+  ~HostLink();
+};
+}
+}  // namespace mfm
 
 struct mfm_ctx {
   mfm_params p;
@@ -21,6 +34,11 @@ struct mfm_ctx {
   // pinned host staging for tables and results
   char* hbuf = nullptr;
   size_t hbuf_bytes = 0;
+  // host-buffer entry points: the pinned pipeline and U's place on the device
+  mfm::host::HostLink link;
+  double* host_u = nullptr;
+  size_t host_u_bytes = 0;
+  bool host_busy = false;  // host_u is the state of a running update
   size_t fsize() const { return p.precision == MFM_PREC_FP32_FLUX ? 4 : 8; }
   // optional per-kernel timing, accumulated per stage and kernel kind
   mfm::KernelTimer* timer = nullptr;
@@ -147,6 +165,15 @@ struct PatchIn {
 int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
               double* new_dt, int* min_cell, double* level_dt, int* min_patch,
               hipStream_t s, const FixedScratch* fixed = nullptr, bool separate = false);
+// A part of a copy: [off, off + bytes) of the host and of the device buffer.
+struct CopySeg {
+  size_t off, bytes;
+};
+// Copies the segments between pageable (or pinned) host memory and the device,
+// large copies through the link's pinned buffers; returns when they are done.
+// Ordered after the null stream's work.
+hipError_t host_copy(HostLink& link, void* dev, void* host, const CopySeg* seg, int nseg,
+                     bool to_dev);
 // Resolves, once per device, the address of the fixed scratch of the
 // allocation-free entry point on the context's device (mfm_noalloc.hip).
 int fixed_scratch_setup(mfm_ctx* c);

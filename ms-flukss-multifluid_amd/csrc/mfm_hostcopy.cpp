@@ -1,0 +1,157 @@
+// mfm_hostcopy.cpp -- copies between pageable host memory and the device.
+//
+// A runtime copy of pageable memory moves through the runtime's staging at
+// about 20 GB/s with one host thread.  Here a few threads each take every
+// kThreads-th chunk of a copy through two pinned buffers of their own and a
+// stream of their own: while one chunk is on the link, the thread copies the
+// next between its other buffer and the caller's memory.  The buffers belong
+// to a HostCopier (16 MiB pinned, allocated with its first large copy and
+// freed with it); threads live for one copy.
+//
+// 64^3 cells, 4 fluids (69 MB up, 61 MB down), FP64 RK2, per
+// mfm_patch_update_host call: 7.35 -> 3.24 ms with U's device memory kept
+// between calls; 24 SW/LISM solves of 20 steps, states fetched: 42 -> 37 ms.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstring>
+#include <mutex>
+#include <new>
+#include <system_error>
+#include <thread>
+
+#include "mfm_host.hpp"
+
+namespace mfm {
+namespace host {
+
+namespace {
+constexpr int kThreads = 4, kSlots = 2;
+constexpr size_t kChunk = (size_t)2 << 20;
+constexpr size_t kLeast = (size_t)4 << 20;  // smaller copies: the runtime's
+}  // namespace
+
+struct HostCopier {
+  int device = -1;
+  char* pin = nullptr;  // kThreads x kSlots chunks
+  hipStream_t st[kThreads] = {};
+  hipEvent_t ev[kThreads][kSlots] = {};
+
+  hipError_t open(int dev) {
+    device = dev;
+    hipError_t e = hipHostMalloc((void**)&pin, kThreads * kSlots * kChunk, hipHostMallocDefault);
+    for (int t = 0; t < kThreads && e == hipSuccess; ++t) {
+      e = hipStreamCreateWithFlags(&st[t], hipStreamNonBlocking);
+      for (int q = 0; q < kSlots && e == hipSuccess; ++q)
+        e = hipEventCreateWithFlags(&ev[t][q], hipEventDisableTiming);
+    }
+    return e;
+  }
+  ~HostCopier() {
+    for (int t = 0; t < kThreads; ++t) {
+      for (int q = 0; q < kSlots; ++q)
+        if (ev[t][q]) (void)hipEventDestroy(ev[t][q]);
+      if (st[t]) (void)hipStreamDestroy(st[t]);
+    }
+    if (pin) (void)hipHostFree(pin);
+  }
+
+  // thread t's chunks of the segments, in their order
+  hipError_t run(int t, char* dev, char* host, const CopySeg* seg, int nseg, bool to_dev) {
+    hipError_t e = hipSetDevice(device);
+    size_t out_off[kSlots] = {}, out_len[kSlots] = {};  // device to host: chunks on the link
+    long turn = 0, mine = 0;
+    auto slot = [&](long m) { return pin + ((size_t)t * kSlots + (size_t)(m % kSlots)) * kChunk; };
+    auto drain = [&](long m) {  // the slot's chunk has arrived: to the caller
+      const int q = (int)(m % kSlots);
+      if (!out_len[q]) return;
+      const hipError_t r = hipEventSynchronize(ev[t][q]);
+      if (e == hipSuccess) e = r;
+      if (e == hipSuccess) std::memcpy(host + out_off[q], slot(m), out_len[q]);
+      out_len[q] = 0;
+    };
+    for (int s = 0; s < nseg && e == hipSuccess; ++s)
+      for (size_t o = 0; o < seg[s].bytes && e == hipSuccess; o += kChunk, ++turn) {
+        if (turn % kThreads != t) continue;
+        const size_t off = seg[s].off + o, len = std::min(kChunk, seg[s].bytes - o);
+        const int q = (int)(mine % kSlots);
+        if (to_dev) {
+          if (mine >= kSlots) e = hipEventSynchronize(ev[t][q]);
+          if (e != hipSuccess) break;
+          std::memcpy(slot(mine), host + off, len);
+          e = hipMemcpyAsync(dev + off, slot(mine), len, hipMemcpyHostToDevice, st[t]);
+        } else {
+          drain(mine);
+          if (e != hipSuccess) break;
+          e = hipMemcpyAsync(slot(mine), dev + off, len, hipMemcpyDeviceToHost, st[t]);
+          out_off[q] = off;
+          out_len[q] = len;
+        }
+        if (e == hipSuccess) e = hipEventRecord(ev[t][q], st[t]);
+        ++mine;
+      }
+    for (int q = 0; q < kSlots; ++q) drain(mine + q);
+    const hipError_t r = hipStreamSynchronize(st[t]);  // no chunk outlives the call
+    return e == hipSuccess ? r : e;
+  }
+};
+
+HostLink::~HostLink() { delete copier; }
+
+hipError_t host_copy(HostLink& link, void* dev, void* host, const CopySeg* seg, int nseg,
+                     bool to_dev) {
+  size_t total = 0;
+  for (int s = 0; s < nseg; ++s) total += seg[s].bytes;
+  // what the null stream has queued comes first, as with a runtime copy
+  hipError_t e = hipStreamSynchronize(nullptr);
+  if (e != hipSuccess) return e;
+  int cur = 0;
+  e = hipGetDevice(&cur);
+  if (e != hipSuccess) return e;
+  hipPointerAttribute_t at;
+  // pinned, managed or device memory that a caller passed is the runtime's to copy
+  const bool known = hipPointerGetAttributes(&at, host) == hipSuccess &&
+                     at.type != hipMemoryTypeUnregistered;
+  (void)hipGetLastError();  // (pageable memory may be reported as an error)
+  // one copy at a time has the buffers; a second thread's is the runtime's
+  std::unique_lock<std::mutex> lock(link.mu, std::defer_lock);
+  bool own = total >= kLeast && !known && lock.try_lock();
+  if (own && !link.copier) {
+    HostCopier* h = new (std::nothrow) HostCopier();
+    if (h && h->open(cur) == hipSuccess) {
+      link.copier = h;
+    } else {
+      delete h;
+      (void)hipGetLastError();
+    }
+  }
+  HostCopier* hc = link.copier;
+  own = own && hc && hc->device == cur;
+  char* d = static_cast<char*>(dev);
+  char* p = static_cast<char*>(host);
+  if (!own) {
+    for (int s = 0; s < nseg && e == hipSuccess; ++s)
+      e = to_dev ? hipMemcpy(d + seg[s].off, p + seg[s].off, seg[s].bytes, hipMemcpyHostToDevice)
+                 : hipMemcpy(p + seg[s].off, d + seg[s].off, seg[s].bytes, hipMemcpyDeviceToHost);
+    return e;
+  }
+  hipError_t res[kThreads];
+  std::thread th[kThreads];
+  for (int t = 1; t < kThreads; ++t) {
+    auto body = [&, t]() { res[t] = hc->run(t, d, p, seg, nseg, to_dev); };
+    try {
+      th[t] = std::thread(body);
+    } catch (const std::system_error&) {
+      body();  // no thread to be had: its part here
+    }
+  }
+  res[0] = hc->run(0, d, p, seg, nseg, to_dev);
+  for (int t = 1; t < kThreads; ++t)
+    if (th[t].joinable()) th[t].join();
+  for (int t = 0; t < kThreads; ++t)
+    if (res[t] != hipSuccess) return res[t];
+  return hipSuccess;
+}
+
+}  // namespace host
+}  // namespace mfm

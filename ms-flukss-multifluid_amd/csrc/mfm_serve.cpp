@@ -353,7 +353,8 @@ int mfm_server_fetch(mfm_server* s, long id, double* host, size_t bytes) {
   if (!r->U) return sfail(s, MFM_ERR_ARG, "request holds no state");
   const size_t need = (size_t)r->fab.size() * r->C.nc * sizeof(double);
   if (bytes < need) return sfail(s, MFM_ERR_SHAPE, "host buffer too small");
-  hipError_t e = hipMemcpy(host, r->U, need, hipMemcpyDeviceToHost);
+  const CopySeg whole{0, need};
+  hipError_t e = host_copy(s->ctx->link, r->U, host, &whole, 1, false);
   if (e != hipSuccess) return sfail(s, MFM_ERR_DEVICE, std::string("fetch: ") + hipGetErrorString(e));
   return MFM_OK;
 }
