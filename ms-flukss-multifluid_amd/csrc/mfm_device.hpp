@@ -112,18 +112,23 @@ __device__ __forceinline__ T nonneg(T x) {
 // (P. Markstein, IBM J. Res. Dev. 34 (1990) 111-119), which rounds as the
 // division does; a full FP64 division takes eleven instructions with its
 // scaling for extreme exponents, which the densities, sound speeds and
-// pressures divided by here (positive, floored) do not need.  FP32: the plain
-// quotient (one reciprocal, shared by the compiler, and a multiply).
+// pressures divided by here (positive, floored) do not need.  FP32: the
+// hardware's reciprocal and a multiply, which is what a division is in the
+// FP32 build but for its rescaling of denominators above 2^96 (four more
+// instructions per quotient, of use only above 2^126, where the reciprocal is
+// no normal number).
 // Roe's FP64 flux has some 35 quotients over 11 denominators: 162 instead of
 // 198 registers (3 wavefronts per SIMD instead of 2), the same bits; per step
 // Brio-Wu 800 84 -> 77 us, Orszag-Tang 512^2 with GLM 153 -> 145 us, 512 x 512 x
 // 32 with characteristic slopes 5.33 -> 4.96 ms, four-fluid 128^3 3.27 -> 3.09 ms.
 template <typename T>
-struct Denom {
-  T b;
-  __device__ __forceinline__ explicit Denom(T d) : b(d) {}
-  __device__ __forceinline__ Denom(T d, double) : b(d) {}
-  __device__ __forceinline__ T operator()(T a) const { return a / b; }
+struct Denom;
+template <>
+struct Denom<float> {
+  float r;
+  __device__ __forceinline__ explicit Denom(float d) : r(__builtin_amdgcn_rcpf(d)) {}
+  __device__ __forceinline__ Denom(float, double inv) : r((float)inv) {}
+  __device__ __forceinline__ float operator()(float a) const { return a * r; }
 };
 template <>
 struct Denom<double> {
@@ -142,6 +147,15 @@ struct Denom<double> {
 };
 
 // ------------------------------------------------------------ limiters --
+// The smaller of two FP32 slopes of one sign, zero where the signs differ: the
+// median of the two and zero.  A NaN in b stays one (the median drops it):
+// a slope towards a NaN cell stays an error that the time step reports.
+// Minmod 6 instead of 10 instructions, van Leer without branches.
+__device__ __forceinline__ float minmod32(float a, float b) {
+  const float m = __builtin_amdgcn_fmed3f(a, b, 0.f);
+  return b != b ? b : m;
+}
+
 // src/reconstructionF.ChF: face values of a cell (left = W-, right = W+)
 // from its neighbours wl, wr along the sweep direction.
 template <typename T>
@@ -151,21 +165,32 @@ __device__ __forceinline__ void limit(int lim, T wl, T w0, T wr, T& left,
   const T z = T(0), h = T(0.5);
   switch (lim) {
     case MFM_LIM_MINMOD: {  // minmod, :126-155
-      T s = copysign(T(1), dWR);
-      T m = s * tmax(z, tmin(fabs(dWR), s * dWL));
-      T sl = h * m;
-      left = w0 - sl; right = w0 + sl;
+      if constexpr (std::is_same<T, float>::value) {
+        const float sl = 0.5f * minmod32(dWR, dWL);
+        left = w0 - sl; right = w0 + sl;
+      } else {
+        T s = copysign(T(1), dWR);
+        T m = s * tmax(z, tmin(fabs(dWR), s * dWL));
+        T sl = h * m;
+        left = w0 - sl; right = w0 + sl;
+      }
       return;
     }
     case MFM_LIM_VANLEER: {  // :794-841 (kappa = 1/3)
-      if (dWL * dWR <= z) { left = w0; right = w0; return; }
       const T BT = T((3.0 - 1.0 / 3.0) / (1.0 - 1.0 / 3.0));
       const T SL1 = T(0.25 * (1.0 - 1.0 / 3.0)), SL2 = T(0.25 * (1.0 + 1.0 / 3.0));
-      T SL = tmin(fabs(dWR), fabs(BT * dWL));
-      T SR = tmin(fabs(dWL), fabs(BT * dWR));
-      T pl = SL1 * SL + SL2 * SR, pr = SL1 * SR + SL2 * SL;
-      if (dWR < z) { pl = -pl; pr = -pr; }
-      left = w0 - pl; right = w0 + pr;
+      if constexpr (std::is_same<T, float>::value) {
+        const float SL = minmod32(dWR, BT * dWL), SR = minmod32(dWL, BT * dWR);
+        left = w0 - (SL1 * SL + SL2 * SR);
+        right = w0 + (SL1 * SR + SL2 * SL);
+      } else {
+        if (dWL * dWR <= z) { left = w0; right = w0; return; }
+        T SL = tmin(fabs(dWR), fabs(BT * dWL));
+        T SR = tmin(fabs(dWL), fabs(BT * dWR));
+        T pl = SL1 * SL + SL2 * SR, pr = SL1 * SR + SL2 * SL;
+        if (dWR < z) { pl = -pl; pr = -pr; }
+        left = w0 - pl; right = w0 + pr;
+      }
       return;
     }
     case MFM_LIM_MC: {  // :622-662
@@ -765,98 +790,43 @@ __device__ __forceinline__ void roe_flux(const Consts& C, const MState<T>& L,
   const T sp85 = two * als * sqPiRho * c * hzz, sp87 = -two * alf * sqPiRho * c * hzz;
 
   T ra1, ra2, ra3, ra4, ra5, ra6, ra7, ra8;
-  if constexpr (std::is_same<T, float>::value) {
-    // FP32: |Lambda| = A1 I + D.  The A1 part is A1 times the conserved
-    // jumps (R L = I); only D = |Lambda| - A1 I goes through the
-    // eigenvectors.  With the reference's form, the entropy wave and the
-    // acoustic waves carry opposite dp/c^2 terms that cancel, which at
-    // large Mach number (c^2 << u^2, e.g. a pressure on its floor) FP32
-    // cannot resolve.  Pairs of waves are combined as half-sums and
-    // half-differences of D, each formed without cancellation.
-    const T del = T(C.del2) * (fabs(U) + fabs(V) + fabs(W) + af);
-    auto fix = [&](T e) -> T {
-      const T zz = fabs(e);
-      return zz >= del ? zz : half * (zz * zz + del * del) / del;
-    };
-    auto fixdiff = [&](T sh) -> T {  // fix(U + sh) - fix(U)
-      const T e1 = U + sh, z1 = fabs(e1), z0 = fabs(U);
-      if (z1 >= del && z0 >= del) {
-        if ((e1 >= zero) == (U >= zero)) return U >= zero ? sh : -sh;
-        return z1 - z0;
-      }
-      if (z1 < del && z0 < del) return half * sh * (U + U + sh) / del;
-      return fix(e1) - fix(U);
-    };
-    const T d3 = fixdiff(b), d4 = fixdiff(-b), d5 = fixdiff(af), d6 = fixdiff(-af);
-    const T d7 = fixdiff(as), d8 = fixdiff(-as);
-    const T Pa = -hzs * du3 + hys * du4, Qa = q7 * du7 + (-q8) * du8;
-    const T Xf = so52 * du2 + so53 * du3 + so54 * du4;
-    const T Yf = so55 * du5 + so57 * du7 + so58 * du8;
-    const T Xs = so72 * du2 + so73 * du3 + so74 * du4;
-    const T Ys = so75 * du5 + so77 * du7 + so78 * du8;
-    const T l3 = d3 * (Pa + Qa), l4 = d4 * (Pa - Qa);
-    const T s56 = (d5 - d6) * Xf + (d5 + d6) * Yf, m56 = (d5 + d6) * Xf + (d5 - d6) * Yf;
-    const T s78 = (d7 - d8) * Xs + (d7 + d8) * Ys, m78 = (d7 + d8) * Xs + (d7 - d8) * Ys;
-    ra1 = ra_f * s56 + ra_s * s78;
-    ra2 = aff * m56 + ass * m78;
-    ra3 = -hzs * (l3 + l4) + sp35 * m56 + sp37 * m78;
-    ra4 = hys * (l3 + l4) + sp45 * m56 + sp47 * m78;
-    ra5 = sp55 * s56 + sp57 * s78;
-    ra7 = sp73 * (l3 - l4) + sp75 * s56 + sp77 * s78;
-    ra8 = sp83 * (l3 - l4) + sp85 * s56 + sp87 * s78;
-    ra6 = zero;
+  const T so15 = -ic;
+  const T lu1 = A1 * (du1 + so15 * du5);
+  const T lu3 = A3 * (-hzs * du3 + hys * du4 + q7 * du7 + (-q8) * du8);
+  const T lu4 = A4 * (-hzs * du3 + hys * du4 + (-q7) * du7 + q8 * du8);
+  const T lu5 = A5 * (so52 * du2 + so53 * du3 + so54 * du4 + so55 * du5 +
+                      so57 * du7 + so58 * du8);
+  const T lu6 = A6 * ((-so52) * du2 + (-so53) * du3 + (-so54) * du4 +
+                      so55 * du5 + so57 * du7 + so58 * du8);
+  const T lu7 = A7 * (so72 * du2 + so73 * du3 + so74 * du4 + so75 * du5 +
+                      so77 * du7 + so78 * du8);
+  const T lu8 = A8 * ((-so72) * du2 + (-so73) * du3 + (-so74) * du4 +
+                      so75 * du5 + so77 * du7 + so78 * du8);
+
+  ra1 = lu1 + ra_f * lu5 + ra_f * lu6 + ra_s * lu7 + ra_s * lu8;
+  ra2 = aff * lu5 + (-aff) * lu6 + ass * lu7 + (-ass) * lu8;
+  ra3 = -hzs * lu3 + (-hzs) * lu4 + sp35 * lu5 + (-sp35) * lu6 + sp37 * lu7 +
+          (-sp37) * lu8;
+  ra4 = hys * lu3 + hys * lu4 + sp45 * lu5 + (-sp45) * lu6 + sp47 * lu7 +
+          (-sp47) * lu8;
+  ra5 = sp55 * lu5 + sp55 * lu6 + sp57 * lu7 + sp57 * lu8;
+  ra7 = sp73 * lu3 + (-sp73) * lu4 + sp75 * lu5 + sp75 * lu6 + sp77 * lu7 +
+          sp77 * lu8;
+  ra8 = sp83 * lu3 + (-sp83) * lu4 + sp85 * lu5 + sp85 * lu6 + sp87 * lu7 +
+          sp87 * lu8;
+  ra6 = zero;
+  if constexpr (!seven) {
+    ra6 = A1 * du6;  // lu2 = |U| * du6, sp62 = 1
+    ra5 = ra1 * kk + Rho * (U * ra2 + V * ra3 + W * ra4) + byHg(ra5) +
+          c4 * (BX * ra6 + BY * ra7 + BZ * ra8);
+  } else {
     ra5 = ra1 * kk + Rho * (U * ra2 + V * ra3 + W * ra4) + byHg(ra5) +
           c4 * (BY * ra7 + BZ * ra8);
-    ra2 = U * ra1 + Rho * ra2;
-    ra3 = V * ra1 + Rho * ra3;
-    ra4 = W * ra1 + Rho * ra4;
-    ra1 = ra1 + A1 * dcons[0];
-    ra2 = ra2 + A1 * dcons[1];
-    ra3 = ra3 + A1 * dcons[2];
-    ra4 = ra4 + A1 * dcons[3];
-    ra5 = ra5 + A1 * dcons[4];
-    if constexpr (!seven) ra6 = A1 * dcons[5];
-    ra7 = ra7 + A1 * dcons[6];
-    ra8 = ra8 + A1 * dcons[7];
-  } else {
-    const T so15 = -ic;
-    const T lu1 = A1 * (du1 + so15 * du5);
-    const T lu3 = A3 * (-hzs * du3 + hys * du4 + q7 * du7 + (-q8) * du8);
-    const T lu4 = A4 * (-hzs * du3 + hys * du4 + (-q7) * du7 + q8 * du8);
-    const T lu5 = A5 * (so52 * du2 + so53 * du3 + so54 * du4 + so55 * du5 +
-                        so57 * du7 + so58 * du8);
-    const T lu6 = A6 * ((-so52) * du2 + (-so53) * du3 + (-so54) * du4 +
-                        so55 * du5 + so57 * du7 + so58 * du8);
-    const T lu7 = A7 * (so72 * du2 + so73 * du3 + so74 * du4 + so75 * du5 +
-                        so77 * du7 + so78 * du8);
-    const T lu8 = A8 * ((-so72) * du2 + (-so73) * du3 + (-so74) * du4 +
-                        so75 * du5 + so77 * du7 + so78 * du8);
-
-    ra1 = lu1 + ra_f * lu5 + ra_f * lu6 + ra_s * lu7 + ra_s * lu8;
-    ra2 = aff * lu5 + (-aff) * lu6 + ass * lu7 + (-ass) * lu8;
-    ra3 = -hzs * lu3 + (-hzs) * lu4 + sp35 * lu5 + (-sp35) * lu6 + sp37 * lu7 +
-            (-sp37) * lu8;
-    ra4 = hys * lu3 + hys * lu4 + sp45 * lu5 + (-sp45) * lu6 + sp47 * lu7 +
-            (-sp47) * lu8;
-    ra5 = sp55 * lu5 + sp55 * lu6 + sp57 * lu7 + sp57 * lu8;
-    ra7 = sp73 * lu3 + (-sp73) * lu4 + sp75 * lu5 + sp75 * lu6 + sp77 * lu7 +
-            sp77 * lu8;
-    ra8 = sp83 * lu3 + (-sp83) * lu4 + sp85 * lu5 + sp85 * lu6 + sp87 * lu7 +
-            sp87 * lu8;
-    ra6 = zero;
-    if constexpr (!seven) {
-      ra6 = A1 * du6;  // lu2 = |U| * du6, sp62 = 1
-      ra5 = ra1 * kk + Rho * (U * ra2 + V * ra3 + W * ra4) + byHg(ra5) +
-            c4 * (BX * ra6 + BY * ra7 + BZ * ra8);
-    } else {
-      ra5 = ra1 * kk + Rho * (U * ra2 + V * ra3 + W * ra4) + byHg(ra5) +
-            c4 * (BY * ra7 + BZ * ra8);
-    }
-
-    ra2 = U * ra1 + Rho * ra2;
-    ra3 = V * ra1 + Rho * ra3;
-    ra4 = W * ra1 + Rho * ra4;
   }
+
+  ra2 = U * ra1 + Rho * ra2;
+  ra3 = V * ra1 + Rho * ra3;
+  ra4 = W * ra1 + Rho * ra4;
 
   const T fl1 = RUL, fr1 = RUR;
   const T fl2 = L.u * RUL - L.bx * L.bx * c4 + PL;
@@ -873,6 +843,180 @@ __device__ __forceinline__ void roe_flux(const Consts& C, const MState<T>& L,
   out[3] = half * (fl4 + fr4 + ra4);
   out[4] = half * (fl5 + fr5 + ra5);
   out[5] = seven ? zero : half * (zero + zero + ra6);
+  out[6] = half * (fl7 + fr7 + ra7);
+  out[7] = half * (fl8 + fr8 + ra8);
+}
+
+// RIEMANNF / RIEMANN7F of the FP32-flux build: roe_flux's states, averages and
+// waves, the dissipation in the form that FP32 resolves.
+//
+// |Lambda| = A1 I + D: the A1 part is A1 times the conserved jumps (R L = I);
+// only D = |Lambda| - A1 I goes through the eigenvectors.  With the
+// reference's form, the entropy wave and the acoustic waves carry opposite
+// dp/c^2 terms that cancel, which at large Mach number (c^2 << u^2, e.g. a
+// pressure on its floor) FP32 cannot resolve.  The two waves U + s and U - s of a
+// kind enter as the half-sum and half-difference of their D, each formed without
+// cancellation (jump_pair).
+//
+// The kernels around it are bound by VALU issue, so the eigenvector products
+// are grouped by their shared factors, selects take the place of branches and
+// a reciprocal that several quotients share is formed once.  With the limiters
+// and quotients of this build (minmod32, Denom): 256^3, four fluids, the plasma's
+// tile kernel 1.29 -> 1.04 ms (720 -> 520 VALU instructions per face), the neutrals'
+// 1.33 -> 1.19, a step 11.9 -> 11.2 ms; 91 x 75 x 53, two fluids, van Leer, the face
+// kernel 39 -> 24 us.  Errors against the FP64 flux over random states (smooth, jumps,
+// Mach 20, cold, without tangential field) equal the ungrouped form's.
+template <bool seven>
+__device__ __forceinline__ void roe_flux32(const Consts& C, const MState<float>& L,
+                                           const MState<float>& R, float* out) {
+  using T = float;
+  const T half = 0.5f, one = 1.f, zero = 0.f, two = 2.f;
+  const T g = (T)C.gamma, hg = (T)C.hgamma;
+  const T c4 = (T)k1_4PI, c8 = (T)k1_8PI, rs2 = (T)kSQRT_2;
+  const Denom<T> byHg(hg, C.invhgamma), byRhoL(L.rho), byRhoR(R.rho);
+
+  const T RUL = L.rho * L.u, RVL = L.rho * L.v, RWL = L.rho * L.w;
+  const T BxBL = c8 * (L.bx * L.bx + L.by * L.by + L.bz * L.bz);
+  const T RUxUL = half * (RUL * L.u + RVL * L.v + RWL * L.w);
+  const T PL = L.p + BxBL;
+  const T EL = byHg(L.p) + RUxUL + BxBL;
+  const T AL2 = byRhoL(g * L.p);
+  const T RUR = R.rho * R.u, RVR = R.rho * R.v, RWR = R.rho * R.w;
+  const T BxBR = c8 * (R.bx * R.bx + R.by * R.by + R.bz * R.bz);
+  const T RUxUR = half * (RUR * R.u + RVR * R.v + RWR * R.w);
+  const T PR = R.p + BxBR;
+  const T ER = byHg(R.p) + RUxUR + BxBR;
+  const T AR2 = byRhoR(g * R.p);
+
+  T Rho, U, V, W, BX, BY, BZ, BX2, BYZ2, BxBH, kk, cc;
+  if (C.iAveraging == 1) {
+    const T HL = byRhoL(EL + PL), HR = byRhoR(ER + PR);
+    const T cL = __builtin_amdgcn_rcpf(one + tsqrt(byRhoL(R.rho)));
+    const T cR = one - cL;
+    Rho = R.rho * cL + L.rho * cR;
+    U = L.u * cL + R.u * cR;
+    V = L.v * cL + R.v * cR;
+    W = L.w * cL + R.w * cR;
+    const T HAV = HL * cL + HR * cR;
+    BX = R.bx * cL + L.bx * cR;
+    BY = R.by * cL + L.by * cR;
+    BZ = R.bz * cL + L.bz * cR;
+    const T BXAV = half * (L.bx + R.bx);
+    BX2 = BXAV * BXAV;
+    BYZ2 = BY * BY + BZ * BZ;
+    BxBH = c8 * (BX2 + BYZ2);
+    kk = half * (U * U + V * V + W * W);
+    const T dbx = R.bx - L.bx, dby = R.by - L.by, dbz = R.bz - L.bz;
+    const T X = byRhoL(c8 * (dbx * dbx + dby * dby + dbz * dbz) * cL * cL);
+    cc = hg * (HAV - kk - Denom<T>(Rho)(c4 * (BX * BXAV + BYZ2))) + (two - g) * X;
+  } else {
+    Rho = half * (L.rho + R.rho);
+    U = half * (L.u + R.u); V = half * (L.v + R.v); W = half * (L.w + R.w);
+    BX = half * (L.bx + R.bx); BY = half * (L.by + R.by); BZ = half * (L.bz + R.bz);
+    const T P = half * (PL + PR);
+    BX2 = BX * BX;
+    BYZ2 = BY * BY + BZ * BZ;
+    BxBH = c8 * (BX2 + BYZ2);
+    kk = half * (U * U + V * V + W * W);
+    cc = Denom<T>(Rho)(g * (P - BxBH));
+  }
+  const Denom<T> byRho(Rho);
+  const T bb = byRho(c4 * BX2);
+  const T ccmi = tmin(AR2, AL2), ccma = tmax(AL2, AR2);
+  cc = cc < ccmi ? ccmi : cc;
+  cc = cc > ccma ? ccma : cc;
+  const T b = tsqrt(bb), c = tsqrt(cc);
+
+  // (BY, BZ) / |BYZ| and the fast and slow speeds
+  const T sB = (T)C.smallB;
+  const bool noBt = BYZ2 < sB * sB;
+  const Denom<T> byHyz(tsqrt(BYZ2));
+  const T hyy = noBt ? rs2 : byHyz(BY), hzz = noBt ? rs2 : byHyz(BZ);
+  const T szb = cc + byRho(BxBH + BxBH);
+  const T hh = tsqrt(nonneg(szb * szb - 4.f * cc * bb));
+  T aas = half * (szb - hh), aaf = half * (szb + hh);
+  aas = aas <= zero ? zero : (aas >= cc ? cc : aas);
+  aaf = aaf <= cc ? cc : aaf;
+  const bool bOver = bb > cc;
+  aaf = noBt ? (bOver ? bb : cc) : aaf;
+  aas = noBt ? (bOver ? cc : bb) : aas;
+  const T af = tsqrt(aaf), as = tsqrt(aas);
+  const T dfs = aaf - aas, cs = cc - aas, fc = aaf - cc;
+  const Denom<T> byDfs(dfs);
+  T alf = tsqrt(byDfs(cs)), als = tsqrt(byDfs(fc));
+  const bool fast = dfs < 1.0e-8f, slow = !fast && cs <= zero, fast2 = fast || fc <= zero;
+  alf = slow ? zero : (fast2 ? one : alf);
+  als = slow ? one : (fast2 ? zero : als);
+  const T sih = BX >= zero ? one : -one;
+
+  // |lambda| with the entropy fix: A1 = |U| fixed, and per kind of wave of speed
+  // s the sum and the difference of D(U + s) and D(U - s)
+  const T del = (T)C.del2 * (fabs(U) + fabs(V) + fabs(W) + af);
+  const T hdel = half * del, hid = half * __builtin_amdgcn_rcpf(del);
+  const T aU = fabs(U), sU = U >= zero ? one : -one;
+  const bool ge = aU >= del;
+  const T A1 = ge ? aU : aU * aU * hid + hdel;
+  auto jump_pair = [&](T s, T& sum, T& dif) {
+    const T tp = aU + s, tm = aU - s, zm = fabs(tm);
+    const T up = ge ? s : (tp >= del ? tp - A1 : s * (aU + tp) * hid);
+    const T fm = zm >= del ? zm - A1 : zm * zm * hid + hdel - A1;
+    const T dn = ge ? (tm >= del ? -s : fm) : (zm < del ? -s * (aU + tm) * hid : fm);
+    sum = up + dn;
+    dif = sU * (up - dn);
+  };
+  T sa, da, sf, df, ss, ds;
+  jump_pair(b, sa, da);
+  jump_pair(af, sf, df);
+  jump_pair(as, ss, ds);
+
+  T du[8], dcons[8];
+  roe_jumps<T, seven>(C, L, R, byRho, U, V, W, BX, BY, BZ, kk, du, dcons);
+  const T sq = tsqrt((T)kPI * Rho), sq2 = two * rs2 * sq;
+  const T isq = __builtin_amdgcn_rcpf(sq), ic = __builtin_amdgcn_rcpf(cc);
+  const T hic = half * ic, aff = alf * af, ass = als * as;
+  // left eigenvectors times the jumps
+  const T Pa = rs2 * (hyy * du[3] - hzz * du[2]);
+  const T Qa = half * rs2 * isq * sih * (hzz * du[6] - hyy * du[7]);
+  const T vt = sih * (hyy * du[2] + hzz * du[3]);
+  const T Xf = hic * (aff * du[1] - ass * vt), Xs = hic * (ass * du[1] + aff * vt);
+  const T P5 = byRho(hic * du[4]), Bt = 0.25f * ic * c * isq * (hyy * du[6] + hzz * du[7]);
+  const T Yf = alf * P5 + als * Bt, Ys = als * P5 - alf * Bt;
+  // D of the waves, and the right eigenvectors
+  const T lp = rs2 * (sa * Pa + da * Qa), lm = sih * sq2 * (sa * Qa + da * Pa);
+  const T s56 = df * Xf + sf * Yf, m56 = sf * Xf + df * Yf;
+  const T s78 = ds * Xs + ss * Ys, m78 = ss * Xs + ds * Ys;
+  const T M = sih * (aff * m78 - ass * m56);
+  const T N = two * sq * c * (als * s56 - alf * s78);
+  T ra1 = Rho * (alf * s56 + als * s78);
+  T ra2 = aff * m56 + ass * m78;
+  T ra3 = hyy * M - hzz * lp;
+  T ra4 = hzz * M + hyy * lp;
+  T ra7 = hzz * lm + hyy * N;
+  T ra8 = hzz * N - hyy * lm;
+  T ra5 = ra1 * kk + Rho * (U * ra2 + V * ra3 + W * ra4) + byHg(cc * ra1) +
+          c4 * (BY * ra7 + BZ * ra8);
+  ra2 = U * ra1 + Rho * ra2 + A1 * dcons[1];
+  ra3 = V * ra1 + Rho * ra3 + A1 * dcons[2];
+  ra4 = W * ra1 + Rho * ra4 + A1 * dcons[3];
+  ra1 = ra1 + A1 * dcons[0];
+  ra5 = ra5 + A1 * dcons[4];
+  ra7 = ra7 + A1 * dcons[6];
+  ra8 = ra8 + A1 * dcons[7];
+
+  const T fl2 = L.u * RUL - L.bx * L.bx * c4 + PL;
+  const T fr2 = R.u * RUR - R.bx * R.bx * c4 + PR;
+  const T fl3 = L.u * RVL - L.bx * L.by * c4, fr3 = R.u * RVR - R.bx * R.by * c4;
+  const T fl4 = L.u * RWL - L.bx * L.bz * c4, fr4 = R.u * RWR - R.bx * R.bz * c4;
+  const T fl5 = L.u * (EL + PL) - L.bx * (L.u * L.bx + L.v * L.by + L.w * L.bz) * c4;
+  const T fr5 = R.u * (ER + PR) - R.bx * (R.u * R.bx + R.v * R.by + R.w * R.bz) * c4;
+  const T fl7 = L.u * L.by - L.bx * L.v, fr7 = R.u * R.by - R.bx * R.v;
+  const T fl8 = L.u * L.bz - L.bx * L.w, fr8 = R.u * R.bz - R.bx * R.w;
+  out[0] = half * (RUL + RUR + ra1);
+  out[1] = half * (fl2 + fr2 + ra2);
+  out[2] = half * (fl3 + fr3 + ra3);
+  out[3] = half * (fl4 + fr4 + ra4);
+  out[4] = half * (fl5 + fr5 + ra5);
+  out[5] = seven ? zero : half * (A1 * dcons[5]);
   out[6] = half * (fl7 + fr7 + ra7);
   out[7] = half * (fl8 + fr8 + ra8);
 }
@@ -898,8 +1042,9 @@ __device__ __forceinline__ void rusanov_flux(const Consts& C,
   const T BXR4 = R.bx * c4;
   T Rho, U, BX2, BxBH, A2;
   if (C.iAveraging == 1) {
-    const T HL = (EL + PL) / L.rho, HR = (ER + PR) / R.rho;
-    const T cL = one / (one + tsqrt(R.rho / L.rho));
+    const Denom<T> byRhoL(L.rho), byRhoR(R.rho);
+    const T HL = byRhoL(EL + PL), HR = byRhoR(ER + PR);
+    const T cL = Denom<T>(one + tsqrt(byRhoL(R.rho)))(one);
     const T cR = one - cL;
     Rho = R.rho * cL + L.rho * cR;
     U = L.u * cL + R.u * cR;
@@ -913,8 +1058,8 @@ __device__ __forceinline__ void rusanov_flux(const Consts& C,
     BxBH = c8 * (BX2 + BYZ2);
     const T kk = half * (U * U + V * V + W * W);
     const T dbx = R.bx - L.bx, dby = R.by - L.by, dbz = R.bz - L.bz;
-    const T X = c8 * (dbx * dbx + dby * dby + dbz * dbz) * cL * cL / L.rho;
-    A2 = hg * (HAV - kk - c4 * (BX * BXAV + BYZ2) / Rho) + (two - g) * X;
+    const T X = byRhoL(c8 * (dbx * dbx + dby * dby + dbz * dbz) * cL * cL);
+    A2 = hg * (HAV - kk - Denom<T>(Rho)(c4 * (BX * BXAV + BYZ2))) + (two - g) * X;
   } else {
     Rho = half * (L.rho + R.rho);
     U = half * (L.u + R.u);
