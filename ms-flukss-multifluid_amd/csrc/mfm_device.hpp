@@ -576,9 +576,9 @@ __device__ __forceinline__ void neutral_to_prim(const Consts& C, const double* u
   w[0] = r; w[1] = ax; w[2] = ay; w[3] = az; w[4] = q;
 }
 
+// The plasma (8 components).
 template <class S>
-__device__ __forceinline__ void cons_to_prim(const Consts& C, const double* u,
-                                             double* w) {
+__device__ __forceinline__ void plasma_to_prim(const Consts& C, const double* u, double* w) {
   double rho = u[0];
   if (S::NF > 1) rho = fmaxr(C.smallr, u[0]);
   const double ir = 1.0 / rho;
@@ -589,6 +589,12 @@ __device__ __forceinline__ void cons_to_prim(const Consts& C, const double* u,
   p = fmaxr(C.smallp, p);
   w[0] = rho; w[1] = vx; w[2] = vy; w[3] = vz; w[4] = p;
   w[5] = u[5]; w[6] = u[6]; w[7] = u[7];
+}
+
+template <class S>
+__device__ __forceinline__ void cons_to_prim(const Consts& C, const double* u,
+                                             double* w) {
+  plasma_to_prim<S>(C, u, w);
   if (S::DED) w[8] = u[8];
 #pragma unroll
   for (int f = 1; f < S::NF; ++f)
