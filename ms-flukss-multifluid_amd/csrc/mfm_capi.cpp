@@ -27,21 +27,23 @@ constexpr int kBlk = 256;
 // MFM_STAGE_AUTO.  FP32 fluxes: the face sums for a call whose cells fill this
 // part of their 64 x 8 tiles; else (and in FP64 and for Hancock's corrector)
 // from so many cells on, in 3-D, with one plasma limiter that has a kernel of
-// its own.  Per RK2 step, separate kernels against face sums: FP32, 4 fluids,
-// 80^3 481 / 468 us, 96^3 815 / 759, 128^3 1.82 / 1.67 ms, 192^3 5.87 / 5.11;
-// 2 fluids 96^3 536 / 456 us, 128^3 1.21 / 1.03 ms; 1 fluid 96^3 277 / 296 us, 128^3
-// 681 / 656; FP64, 4 fluids, 96^3 1.31 / 1.37 ms, 128^3 3.01 / 2.88, 160^3 5.80 / 5.40;
-// 2 fluids 128^3 1.83 / 1.84, 160^3 3.46 / 3.39, 1 fluid slower at every size (the
-// plasma tile kernel holds 2 wavefronts per SIMD, the face kernel 3; the
-// gain is the neutral fluids'); Hancock, FP32, 4 fluids 96^3 0.70 / 0.70, 128^3
-// 1.56 / 1.45 ms.
+// its own.  Per RK2 step, separate kernels against face sums (z-chunks as
+// chosen below): FP32, 4 fluids, 64^3 223 / 241 us, 80^3 453 / 410, 96^3 772 / 699, 128^3
+// 1.72 / 1.52 ms, 192^3 5.66 / 4.66; 2 fluids 64^3 169 / 169 us, 80^3 278 / 257, 96^3 505 /
+// 396, 128^3 1.15 / 0.91 ms; 1 fluid 96^3 245 / 252 us, 128^3 621 / 561; FP64, 4 fluids,
+// 96^3 1.31 / 1.37 ms, 128^3 3.01 / 2.85, 160^3 5.80 / 5.40; 2 fluids 128^3 1.83 / 1.84,
+// 160^3 3.46 / 3.39, 1 fluid slower at every size (the plasma tile kernel
+// holds 2 wavefronts per SIMD, the face kernel 3; the gain is the neutral
+// fluids'); Hancock, FP32, 4 fluids 96^3 633 / 610 us, 128^3 1.44 / 1.33 ms, 2 fluids
+// 96^3 391 / 337 us.
 constexpr double kAutoTileFill = 0.75;
-constexpr double kAutoCells = 6.0e5, kAutoCells1 = 2.0e6, kAutoCellsHan = 1.3e6,
+constexpr double kAutoCells = 4.0e5, kAutoCells1 = 2.0e6, kAutoCellsHan = 8.0e5,
                  kAutoCells64 = 2.0e6;
 // Blocks of 512 threads (twice as many of 256) below which the z-chunks get
-// shorter: 64^3, FP32, 2 fluids, chunks of 8 / 4 / 2 / 1 planes 405 / 261 / 204 / 185 us;
-// 96^3 595 / 456 / 454 / 458; 128^3 1079 / 1028 / 1037 / 1080.
-constexpr double kAutoBlocks = 1000.0;
+// shorter: a little more than the 512 that the chip holds of the plasma's.  FP32,
+// 4 fluids, chunks of 8 / 4 / 2 planes: 80^3 466 / 428 / 409 us, 96^3 741 / 700 / 699, 128^3
+// 1582 / 1518 / 1555, 192^3 4663 / 4649 / 4779 (1000 blocks: one plane at 96^3, 724).
+constexpr double kAutoBlocks = 600.0;
 const double eos_mp = 1.67262171e-24, eos_k = 1.3806505e-16;
 
 int fail(mfm_ctx* c, int code, const std::string& m) {
@@ -493,7 +495,7 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
       if (dims == 3 && one_lim && (C0.nf > 1 || (f32 && !han)) && cells >= least)
         mode = MFM_STAGE_SUMMED;
       if (f32 && r256 < r512) sum_block = 256;
-      // shorter z-chunks where the blocks would not fill the chip twice over
+      // shorter z-chunks where the blocks would not fill the chip
       const double planes = sum_block == 512 ? p512 : 0.5 * p256;
       while (tz > 1 && planes < kAutoBlocks * tz) tz /= 2;
     }
