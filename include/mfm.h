@@ -263,7 +263,7 @@ int mfm_ctx_get_timing(mfm_ctx* ctx, int stage, int kind, double* ms,
  * runs the separate kernels in this mode).
  * MFM_STAGE_AUTO (default): per call, the summed stages where they are the
  * faster ones -- in the FP32-flux build when the cells fill at least 3/4 of
- * their 64 x 8 column tiles (12.2 against 13.9-14.2 ms per step on the 256^3
+ * their 64 x 8 column tiles (10.8 against 13.1 ms per step on the 256^3
  * workload), and in either build from a number of cells on that depends on
  * the fluids and the scheme, with shorter z-chunks (tz at most) for small
  * calls -- else the separate kernels; the allocation-free entry point always

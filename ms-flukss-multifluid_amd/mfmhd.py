@@ -415,7 +415,7 @@ class Context:
     def set_stage_kernel(self, mode, tz=8):
         """Kernel structure of RK2 / first-order stages: STAGE_SEPARATE,
         STAGE_FUSED (True), STAGE_SUMMED or STAGE_AUTO (the default: summed
-        where the column tiles are well filled, FP32-flux build); tz =
+        where it is the faster one for the call's size); tz =
         planes per z-chunk of the tile kernels."""
         if isinstance(mode, bool):
             mode = STAGE_FUSED if mode else STAGE_SEPARATE
