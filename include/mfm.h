@@ -501,7 +501,10 @@ int mfm_server_create(const mfm_params* cls, double hbm_budget_bytes,
 int mfm_server_destroy(mfm_server* srv);
 const char* mfm_server_last_error(const mfm_server* srv);
 /* The stage structure of every batch (MFM_STAGE_SEPARATE, the default,
- * MFM_STAGE_SUMMED or MFM_STAGE_FUSED; see mfm_ctx_set_stage_kernel).  A
+ * MFM_STAGE_SUMMED or MFM_STAGE_FUSED; see mfm_ctx_set_stage_kernel; FP64
+ * and Hancock servers run the separate kernels for MFM_STAGE_SUMMED; with
+ * the tile kernels, requests with different plasma limiters go in batches of
+ * their own).  A
  * fixed structure keeps a request's result independent of its batch, so
  * MFM_STAGE_AUTO is refused; so is a change after the first request (its
  * HBM estimate depends on the structure).  No counterpart in the

@@ -504,9 +504,12 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
   const bool fused = mode == MFM_STAGE_FUSED;
   const bool summed = mode == MFM_STAGE_SUMMED;
   if (n <= 0) return fail(c, MFM_ERR_ARG, "empty patch table");
-  for (int r = 1; r < nct; ++r)
+  for (int r = 1; r < nct; ++r) {
     if (Ct[r].dims != C0.dims || Ct[r].nf != C0.nf || Ct[r].dedner != C0.dedner)
       return fail(c, MFM_ERR_ARG, "constants of one batch must share dimension, fluids and GLM");
+    if ((fused || summed) && tile_limiter(Ct[r]) != tile_limiter(C0))
+      return fail(c, MFM_ERR_ARG, "the tile kernels take one plasma limiter per batch");
+  }
   SmallVec<PatchGeo, 1> G;
   G.resize(n);
   size_t off = 0;

@@ -160,6 +160,15 @@ struct PatchIn {
   double dt, dx, time;
 };
 
+// The limiter instance of the tile kernels (k_stage, the face sums) that a
+// patch takes.  A launch has one for all its patches, so the patches of a
+// batch that runs them share it: the limiter a patch gets (and, in the
+// FP32-flux build, the compiler's contraction of it) may not depend on the
+// patches beside it.
+inline int tile_limiter(const Consts& C) {
+  return C.plasma_lim == MFM_LIM_MINMOD || C.plasma_lim == MFM_LIM_VANLEER ? C.plasma_lim : -1;
+}
+
 // separate: MFM_STAGE_AUTO takes the separate kernels (too little memory for
 // the face sums' scratch).
 int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,

@@ -72,6 +72,7 @@ size_t request_bytes(const mfm_params& cls, int mode, const Consts& C, const HBo
   const int dims = C.dims;
   const size_t fs = cls.precision == MFM_PREC_FP32_FLUX ? 4 : 8;
   const size_t cells = (size_t)fab.size();
+  // (mfm_server_set_stage_kernel leaves a tile structure only where it runs)
   const bool tiles = cls.time_approx != MFM_TIME_HANCOCK && !cls.char_reconstruction;
   size_t b = align256(cells * C.nc * 8);          // U
   b += align256(cells * C.nc * 8);                // U*
@@ -79,7 +80,7 @@ size_t request_bytes(const mfm_params& cls, int mode, const Consts& C, const HBo
   if (cls.time_approx == MFM_TIME_HANCOCK) b += align256(cells * C.nc * fs);  // W of U_pred
   if (tiles && mode == MFM_STAGE_FUSED && cls.time_approx == MFM_TIME_RK2)
     b += align256(cells * C.nc * fs);             // W of U*
-  if (!cls.char_reconstruction && mode == MFM_STAGE_SUMMED)
+  if (tiles && mode == MFM_STAGE_SUMMED)
     b += align256(cells * (C.nc + 1) * fs);       // face sums
   HBox v1 = cls.time_approx == MFM_TIME_RK2 ? grow(valid, 2, dims)
             : (cls.time_approx == MFM_TIME_HANCOCK ? grow(valid, 1, dims) : valid);
@@ -160,6 +161,65 @@ int admit(mfm_server* s) {
   return MFM_OK;
 }
 
+// One step of the requests of a batch (their own dt each) in the same launches;
+// ms: wall time, added.
+int step_batch(mfm_server* s, const std::vector<Request*>& batch, double& ms) {
+  const int n = (int)batch.size();
+  std::vector<Consts> Ct(n);
+  std::vector<PatchIn> in(n);
+  std::vector<double> nd(n);
+  std::vector<int> cell(3 * n);
+  for (int q = 0; q < n; ++q) {
+    Request* r = batch[q];
+    Ct[q] = r->C;
+    in[q].U = mfm_fab{r->U, {{r->fab.lo[0], r->fab.lo[1], r->fab.lo[2]}, {r->fab.hi[0], r->fab.hi[1], r->fab.hi[2]}}, r->C.nc};
+    in[q].valid = mfm_box{{r->valid.lo[0], r->valid.lo[1], r->valid.lo[2]}, {r->valid.hi[0], r->valid.hi[1], r->valid.hi[2]}};
+    in[q].F = nullptr;
+    in[q].divB = nullptr;
+    in[q].cidx = q;
+    // AMRLevelIdealMHD::computeNewDt / computeInitialDt: cfl * dt_raw,
+    // growth limited; the first step uses initial_cfl
+    in[q].dt = r->dt_prev > 0.0 ? std::min(r->cfl * r->dt_raw, r->growth * r->dt_prev)
+                                : r->cfl0 * r->dt_raw;
+    in[q].dx = r->dx;
+    in[q].time = r->t;
+    // periodic directions of a one-patch domain wrap onto themselves
+    bool periodic = false;
+    for (int d = 0; d < r->C.dims; ++d) periodic = periodic || !r->C.phys[d];
+    if (periodic) {
+      int ulo[3], un[3], vlo[3], vn[3];
+      for (int d = 0; d < 3; ++d) {
+        ulo[d] = r->fab.lo[d]; un[d] = (int)r->fab.n(d);
+        vlo[d] = r->valid.lo[d]; vn[d] = (int)r->valid.n(d);
+      }
+      hipError_t e = launch_fill_periodic(r->U, ulo, un, r->fab.size(), r->C.nc, vlo, vn,
+                                          r->C.dims, nullptr);
+      if (e != hipSuccess) return sfail(s, MFM_ERR_DEVICE, "periodic fill launch");
+    }
+  }
+  const double t0 = now_ms();
+  const int rc = run_batch(s->ctx, Ct.data(), n, in.data(), n, nd.data(), cell.data(), nullptr,
+                           nullptr, nullptr);
+  ms += now_ms() - t0;
+  if (rc != MFM_OK && rc != MFM_ERR_NUMERIC) return sfail(s, rc, s->ctx->err);
+  for (int q = 0; q < n; ++q) {
+    Request* r = batch[q];
+    r->t += in[q].dt;
+    r->done += 1;
+    s->cell_updates += (double)r->valid.size();
+    const double d = nd[q];
+    if (!(d > 0.0) || std::isnan(d)) {
+      r->state = REQ_FAILED;
+      r->err = "non-positive or NaN time step";
+    } else {
+      r->dt_raw = d;
+      r->dt_prev = in[q].dt;
+      if (r->done >= r->nsteps) r->state = REQ_DONE;
+    }
+  }
+  return MFM_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -200,6 +260,13 @@ int mfm_server_set_stage_kernel(mfm_server* s, int mode) {
     return sfail(s, MFM_ERR_ARG, "the server takes a fixed stage structure (not AUTO)");
   if (!s->all.empty())
     return sfail(s, MFM_ERR_ARG, "set the stage structure before the first request");
+  // The summed stages in the FP32-flux RK2 and first-order builds.  FP64 gives
+  // the same bits either way and the separate kernels' requests are smaller
+  // (no sums in their share of the budget); Hancock runs the separate ones.
+  const mfm_params& p = s->ctx->p;
+  if (mode == MFM_STAGE_SUMMED &&
+      (p.precision != MFM_PREC_FP32_FLUX || p.time_approx == MFM_TIME_HANCOCK))
+    mode = MFM_STAGE_SEPARATE;
   s->ctx->stage_mode = mode;
   return MFM_OK;
 }
@@ -258,62 +325,23 @@ int mfm_server_step(mfm_server* s, int* n_active, int* n_pending, double* iter_m
   if (rc != MFM_OK) return rc;
   double ms = 0.0;
   if (!s->active.empty()) {
-    const int n = (int)s->active.size();
-    std::vector<Consts> Ct(n);
-    std::vector<PatchIn> in(n);
-    std::vector<double> nd(n);
-    std::vector<int> cell(3 * n);
-    for (int q = 0; q < n; ++q) {
-      Request* r = s->active[q];
-      Ct[q] = r->C;
-      in[q].U = mfm_fab{r->U, {{r->fab.lo[0], r->fab.lo[1], r->fab.lo[2]}, {r->fab.hi[0], r->fab.hi[1], r->fab.hi[2]}}, r->C.nc};
-      in[q].valid = mfm_box{{r->valid.lo[0], r->valid.lo[1], r->valid.lo[2]}, {r->valid.hi[0], r->valid.hi[1], r->valid.hi[2]}};
-      in[q].F = nullptr;
-      in[q].divB = nullptr;
-      in[q].cidx = q;
-      // AMRLevelIdealMHD::computeNewDt / computeInitialDt: cfl * dt_raw,
-      // growth limited; the first step uses initial_cfl
-      in[q].dt = r->dt_prev > 0.0 ? std::min(r->cfl * r->dt_raw, r->growth * r->dt_prev)
-                                  : r->cfl0 * r->dt_raw;
-      in[q].dx = r->dx;
-      in[q].time = r->t;
-      // periodic directions of a one-patch domain wrap onto themselves
-      bool periodic = false;
-      for (int d = 0; d < r->C.dims; ++d) periodic = periodic || !r->C.phys[d];
-      if (periodic) {
-        int ulo[3], un[3], vlo[3], vn[3];
-        for (int d = 0; d < 3; ++d) {
-          ulo[d] = r->fab.lo[d]; un[d] = (int)r->fab.n(d);
-          vlo[d] = r->valid.lo[d]; vn[d] = (int)r->valid.n(d);
-        }
-        hipError_t e = launch_fill_periodic(r->U, ulo, un, r->fab.size(), r->C.nc, vlo, vn,
-                                            r->C.dims, nullptr);
-        if (e != hipSuccess) return sfail(s, MFM_ERR_DEVICE, "periodic fill launch");
-      }
+    // one batch, or with the tile kernels one per limiter instance
+    std::vector<std::vector<Request*>> batches;
+    if (s->ctx->stage_mode == MFM_STAGE_SEPARATE) {
+      batches.push_back(s->active);
+    } else {
+      std::map<int, std::vector<Request*>> by;
+      for (Request* r : s->active) by[tile_limiter(r->C)].push_back(r);
+      for (auto& kv : by) batches.push_back(kv.second);
     }
-    const double t0 = now_ms();
-    rc = run_batch(s->ctx, Ct.data(), n, in.data(), n, nd.data(), cell.data(), nullptr, nullptr,
-                   nullptr);
-    ms = now_ms() - t0;
-    if (rc != MFM_OK && rc != MFM_ERR_NUMERIC) return sfail(s, rc, s->ctx->err);
-    std::vector<Request*> keep;
-    for (int q = 0; q < n; ++q) {
-      Request* r = s->active[q];
-      r->t += in[q].dt;
-      r->done += 1;
-      s->cell_updates += (double)r->valid.size();
-      const double d = nd[q];
-      if (!(d > 0.0) || std::isnan(d)) {
-        r->state = REQ_FAILED;
-        r->err = "non-positive or NaN time step";
-      } else {
-        r->dt_raw = d;
-        r->dt_prev = in[q].dt;
-        if (r->done >= r->nsteps) r->state = REQ_DONE;
-      }
-      if (r->state == REQ_ACTIVE) keep.push_back(r);
+    for (const std::vector<Request*>& batch : batches) {
+      rc = step_batch(s, batch, ms);
+      if (rc != MFM_OK) break;
     }
-    s->active.swap(keep);
+    s->active.erase(std::remove_if(s->active.begin(), s->active.end(),
+                                   [](const Request* r) { return r->state != REQ_ACTIVE; }),
+                    s->active.end());
+    if (rc != MFM_OK) return rc;
     s->iter_ms.push_back(ms);
     s->busy_ms += ms;
   }
