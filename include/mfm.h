@@ -257,7 +257,8 @@ int mfm_ctx_get_timing(mfm_ctx* ctx, int stage, int kind, double* ms,
  * the face-flux differences summed over the directions, or in the FP64 build
  * the state with the directions applied one after the other (the separate
  * kernels' bits); k_update finishes the stage from those.  The Hancock
- * corrector takes it too.  MFM_STAGE_FUSED: one tile kernel per stage solves
+ * corrector takes it too.  The FP32-flux build keeps the sums in FP32, in FP64
+ * for Hancock and for what AUTO takes from the separate kernels by size.  MFM_STAGE_FUSED: one tile kernel per stage solves
  * every face and updates the cells; the face fluxes never reach HBM, but its
  * register budget makes it slower on the 256^3 workload (the Hancock scheme
  * runs the separate kernels in this mode).

@@ -471,6 +471,7 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
       (fixed && mode == MFM_STAGE_SUMMED && (han || !f32)))
     mode = MFM_STAGE_SEPARATE;
   const bool choose = mode == MFM_STAGE_AUTO;
+  bool filled = false;  // the boxes fill 64 x 8 tiles
   int sum_block = f32 ? 512 : 256;
   int tz = std::max(1, c->stage_tz);
   const int slots256 = sum_slots(256, f32 ? 4 : 8, C0.dedner);
@@ -488,7 +489,8 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
         if (f32) sum_rounds(v, t512.of(v), 512, r512, p512);
         sum_rounds(v, t256.of(v), 256, r256, p256);
       }
-      if (f32 && !han && slots > 0.0 && cells >= kAutoTileFill * slots) mode = MFM_STAGE_SUMMED;
+      filled = slots > 0.0 && cells >= kAutoTileFill * slots;
+      if (f32 && !han && filled) mode = MFM_STAGE_SUMMED;
       const bool one_lim = C0.plasma_lim == MFM_LIM_MINMOD || C0.plasma_lim == MFM_LIM_VANLEER;
       const double least = f32 ? (han ? kAutoCellsHan : (C0.nf > 1 ? kAutoCells : kAutoCells1))
                                : (C0.nf > 2 ? kAutoCells64 : 2.0 * kAutoCells64);
@@ -503,6 +505,10 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
   TileCache tiles{sum_block, sum_block == 512 ? sum_slots(512, 4, 0) : slots256, {}};
   const bool fused = mode == MFM_STAGE_FUSED;
   const bool summed = mode == MFM_STAGE_SUMMED;
+  // FP32 fluxes: the face sums in FP64 where the call's other structure, the
+  // separate kernels, would subtract in FP64; in FP32 for the filled boxes
+  // and the fixed mode, whose sums are FP32 by themselves
+  const bool wide = f32 && summed && (han || (choose && !filled));
   if (n <= 0) return fail(c, MFM_ERR_ARG, "empty patch table");
   for (int r = 1; r < nct; ++r) {
     if (Ct[r].dims != C0.dims || Ct[r].nf != C0.nf || Ct[r].dedner != C0.dedner)
@@ -536,7 +542,7 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
     if (han || (fused && rk2)) off += align256((size_t)ucells * C0.nc * fs);
     // summed stages: the per-cell face sums (NC components + normal B)
     g.off_d = off;
-    if (summed) off += align256((size_t)ucells * (C0.nc + 1) * fs);
+    if (summed) off += align256((size_t)ucells * (C0.nc + 1) * (wide ? 8 : fs));
     for (int d = 0; d < dims; ++d) {
       g.fb[d] = g.vb1;
       g.fb[d].hi[d] += 1;
@@ -813,7 +819,8 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
   int n_stage1 = 0;
   // the whole launch sequence of one update (both stages, dt reduction)
   auto enqueue = [&](hipStream_t st) -> int {
-    auto launch = [&](const StageLists& L, const StepArgs& S) -> hipError_t {
+    auto launch = [&](const StageLists& L, StepArgs S) -> hipError_t {
+      S.wide_sums = wide ? 1 : 0;
       const DevPatch* tp = (S.stage == 1 && rk2) ? dp2 : dp;
       hipError_t e3 = f32 ? launch_stage<float>(C0, ct, tp, L, S, dtp, idp, st, c->timer)
                           : launch_stage<double>(C0, ct, tp, L, S, dtp, idp, st, c->timer);
@@ -865,7 +872,7 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
                                   (long long)off_ct, (long long)off_dtp, (long long)off_idp,
                                   (long long)off_dto, (long long)off_ido, dims, p.time_approx,
                                   p.precision, C0.nf, C0.dedner, c->walk_tile,
-                                  c->walk_xcd, mode, tz, sum_block, walk};
+                                  c->walk_xcd, mode, tz, sum_block, walk, wide};
     for (int l = 0; l < kLists; ++l) {
       key.push_back((long long)off_reg[l]);
       key.push_back((long long)lists[l]->v.size());

@@ -103,6 +103,7 @@ struct StepArgs {
                        // 2: Hancock corrector
   int ghosts_set;      // k_prim: W holds the problem's constant ghost states
                        // from the first RK2 stage
+  int wide_sums;       // FP32 fluxes: D holds the face sums in FP64
 };
 
 // Optional kernel timing: a pair of events brackets every launch on the
