@@ -262,11 +262,13 @@ int mfm_ctx_get_timing(mfm_ctx* ctx, int stage, int kind, double* ms,
  * every face and updates the cells; the face fluxes never reach HBM, but its
  * register budget makes it slower on the 256^3 workload (the Hancock scheme
  * runs the separate kernels in this mode).
- * MFM_STAGE_AUTO (default): per call, the summed stages where they are the
- * faster ones -- in the FP32-flux build when the cells fill at least 3/4 of
- * their 64 x 8 column tiles (10.8 against 13.1 ms per step on the 256^3
- * workload), and in either build from a number of cells on that depends on
- * the fluids and the scheme, with shorter z-chunks (tz at most) for small
+ * MFM_STAGE_AUTO (default): per call, the summed stages in the FP32-flux build
+ * when the cells fill at least 3/4 of their 64 x 8 column tiles (10.8 against
+ * 13.1 ms per step on the 256^3 workload; the smallest of them would be a few
+ * percent faster separate), and in either build from a number of cells on
+ * that depends on the fluids, the scheme and whether the call asks for its
+ * face fluxes (RK2 with F stays separate), where they are the faster ones,
+ * with shorter z-chunks (tz at most) for small
  * calls -- else the separate kernels; the allocation-free entry point always
  * takes the separate kernels.  AUTO decides per call: in the FP32-flux build
  * a patch updated alone and in a level can then take different structures

@@ -25,20 +25,41 @@ namespace host {
 
 constexpr int kBlk = 256;
 // MFM_STAGE_AUTO.  FP32 fluxes: the face sums for a call whose cells fill this
-// part of their 64 x 8 tiles; else (and in FP64 and for Hancock's corrector)
-// from so many cells on, in 3-D, with one plasma limiter that has a kernel of
-// its own.  Per RK2 step, separate kernels against face sums (z-chunks as
-// chosen below): FP32, 4 fluids, 64^3 223 / 241 us, 80^3 453 / 410, 96^3 772 / 699, 128^3
-// 1.72 / 1.52 ms, 192^3 5.66 / 4.66; 2 fluids 64^3 169 / 169 us, 80^3 278 / 257, 96^3 505 /
-// 396, 128^3 1.15 / 0.91 ms; 1 fluid 96^3 245 / 252 us, 128^3 621 / 561; FP64, 4 fluids,
-// 96^3 1.31 / 1.37 ms, 128^3 3.01 / 2.85, 160^3 5.80 / 5.40; 2 fluids 128^3 1.83 / 1.84,
-// 160^3 3.46 / 3.39, 1 fluid slower at every size (the plasma tile kernel
-// holds 2 wavefronts per SIMD, the face kernel 3; the gain is the neutral
-// fluids'); Hancock, FP32, 4 fluids 96^3 633 / 610 us, 128^3 1.44 / 1.33 ms, 2 fluids
-// 96^3 391 / 337 us.
+// part of their 64 x 8 tiles, whatever its size (small ones, 64^3 with four
+// fluids or 96^3 with one, take 3-8 % longer so than by the separate kernels).
+// Else, and in FP64, from so many cells on (auto_cells), in 3-D, with one
+// plasma limiter that has a kernel of its own.
 constexpr double kAutoTileFill = 0.75;
-constexpr double kAutoCells = 4.0e5, kAutoCells1 = 2.0e6, kAutoCellsHan = 8.0e5,
-                 kAutoCells64 = 2.0e6;
+
+// Per call, separate kernels / face sums.
+// FP32 (the sums in FP64, z-chunks as chosen below).  RK2, 2 fluids, 72 x 70 x
+// 90 cells 239 / 241 us, 100 x 91 x 60 289 / 274, 130^3 1173 / 1050, 140 x 200 x 200
+// 2883 / 2571; 4 fluids, 100 x 91 x 60 462 / 468, 130^3 1728 / 1744, 64 boxes of 32^3
+// 2449 / 2268, 161 x 161 x 100 2021 / 1820, 200 x 150 x 130 3043 / 2667; 3 fluids, 130^3
+// 1378 / 1414, 161 x 161 x 100 1609 / 1479.  First order, 2 fluids, 91 x 75 x 70 125 /
+// 129, 90 x 120 x 110 313 / 260; 4 fluids, 130^3 781 / 845, 900 boxes of 16^3 2345 /
+// 2347, 140 x 200 x 200 1924 / 1938.  Hancock, 2 fluids, 300 boxes of 16^3 1027 /
+// 993, 130^3 930 / 873; 4 fluids, 130^3 1454 / 1486, 900 boxes of 16^3 4819 / 4402.
+// 1 fluid, 130^3, 631 / 671.
+// FP64, RK2, 4 fluids, 96^3 1.31 / 1.37 ms, 128^3 2.90 / 2.71; 2 fluids, 128^3 1.83 /
+// 1.84, 160^3 3.46 / 3.39; 1 fluid slower at every size (the plasma tile kernel
+// holds 2 wavefronts per SIMD, the face kernel 3; the gain is the neutral
+// fluids').  Hancock, 4 fluids, 128^3 2.28 / 2.19; first order 1.36 / 1.27.
+// With the caller's fluxes the tile kernels write every face as well (those
+// between tiles twice) and RK2's second stage reads them back: RK2, FP32, 4
+// fluids, 130^3 2232 / 2739 us, 900 boxes of 16^3 8405 / 9283; 2 fluids, 130^3 1475 /
+// 1683; FP64, 4 fluids, 128^3 3393 / 3916, 512 boxes of 16^3 6933 / 7730; first
+// order, FP64, 64 boxes of 32^3 1801 / 1891; but FP32, 2 fluids, 130^3 792 / 769, and
+// Hancock 1170 / 1143.
+double auto_cells(bool f32, int time, int nf, bool fluxes) {
+  const double none = std::numeric_limits<double>::infinity();
+  const bool rk2 = time == MFM_TIME_RK2, han = time == MFM_TIME_HANCOCK;
+  if (nf == 1 || (fluxes && (rk2 || (!f32 && !han)))) return none;
+  if (!f32) return nf > 2 ? 2.0e6 : 4.0e6;
+  if (nf == 2) return rk2 ? 4.0e5 : 8.0e5;
+  return rk2 ? 2.0e6 : (han ? 3.5e6 : none);
+}
+
 // Blocks of 512 threads (twice as many of 256) below which the z-chunks get
 // shorter: a little more than the 512 that the chip holds of the plasma's.  FP32,
 // 4 fluids, chunks of 8 / 4 / 2 planes: 80^3 466 / 428 / 409 us, 96^3 741 / 700 / 699, 128^3
@@ -479,11 +500,13 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
     mode = MFM_STAGE_SEPARATE;
     if (!fixed && !separate) {
       TileCache t512{512, sum_slots(512, 4, 0), {}}, t256{256, slots256, {}};
+      bool fluxes = false;
       double cells = 0.0, slots = 0.0, r512 = 0.0, r256 = 0.0, p512 = 0.0, p256 = 0.0;
       for (int q = 0; q < n; ++q) {
         if (in[q].cidx < 0 || in[q].cidx >= nct) continue;
         const HBox v = clip(Ct[in[q].cidx], hb(in[q].valid));
         if (v.size() <= 0) continue;
+        fluxes = fluxes || in[q].F;
         cells += (double)v.size();
         slots += (double)((v.n(0) + 63) / 64 * 64) * (double)((v.n(1) + 7) / 8 * 8) * (double)v.n(2);
         if (f32) sum_rounds(v, t512.of(v), 512, r512, p512);
@@ -492,9 +515,7 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
       filled = slots > 0.0 && cells >= kAutoTileFill * slots;
       if (f32 && !han && filled) mode = MFM_STAGE_SUMMED;
       const bool one_lim = C0.plasma_lim == MFM_LIM_MINMOD || C0.plasma_lim == MFM_LIM_VANLEER;
-      const double least = f32 ? (han ? kAutoCellsHan : (C0.nf > 1 ? kAutoCells : kAutoCells1))
-                               : (C0.nf > 2 ? kAutoCells64 : 2.0 * kAutoCells64);
-      if (dims == 3 && one_lim && (C0.nf > 1 || (f32 && !han)) && cells >= least)
+      if (dims == 3 && one_lim && cells >= auto_cells(f32, p.time_approx, C0.nf, fluxes))
         mode = MFM_STAGE_SUMMED;
       if (f32 && r256 < r512) sum_block = 256;
       // shorter z-chunks where the blocks would not fill the chip
