@@ -73,9 +73,10 @@ struct Consts {
 // Square root of the flux kernels.  FP64: the Goldschmidt iteration from the
 // hardware's reciprocal-square-root estimate with two exact-residual
 // corrections (P. Markstein, IA-64 and Elementary Functions, 2000, ch. 9),
-// which rounds as sqrt does, without sqrt's rescaling of arguments below
-// 2^-767: 17 instead of 22 instructions.  Zero and infinity are returned
-// as they are.  Orszag-Tang 512 x 512 x 32 with characteristic slopes 4.94 -> 4.81 ms
+// which rounds as sqrt does for arguments above 2^-960, whose residuals are
+// normal numbers, without sqrt's rescaling of arguments below 2^-767: 17
+// instead of 22 instructions.  Below 2^-960 (a speed under 1e-144) the last bit
+// may differ.  Zero and infinity are returned as they are.  Orszag-Tang 512 x 512 x 32 with characteristic slopes 4.94 -> 4.81 ms
 // per step, the same bits.
 template <typename T>
 __device__ __forceinline__ T tsqrt(T x) { return sqrt(x); }
@@ -106,13 +107,17 @@ __device__ __forceinline__ T nonneg(T x) {
   return x;
 }
 
-// A denominator shared by several quotients.  FP64: its reciprocal once, by
-// Newton-Raphson from the hardware estimate, then three instructions per
-// quotient: q = a r, corrected by the exact remainder, q + (a - q b) r
-// (P. Markstein, IBM J. Res. Dev. 34 (1990) 111-119), which rounds as the
-// division does; a full FP64 division takes eleven instructions with its
-// scaling for extreme exponents, which the densities, sound speeds and
-// pressures divided by here (positive, floored) do not need.  FP32: the
+// A denominator (not negative) shared by several quotients.  FP64: its
+// reciprocal once, by Newton-Raphson from the hardware estimate, then three
+// instructions per quotient: q = a r, corrected by the exact remainder,
+// q - (q b - a) r (P. Markstein, IBM J. Res. Dev. 34 (1990) 111-119), which
+// rounds as the division does; with the remainder's sign taken so, a zero
+// keeps a division's sign too.  A full FP64 division takes eleven instructions
+// with its scaling for extreme exponents, which the densities, sound speeds and
+// pressures divided by here (positive, floored) do not need: without it a
+// quotient may round to the neighbour where the remainder underflows (|a| below
+// 2^-960), and is a NaN where the denominator is zero or infinite, its
+// reciprocal no normal number, or the quotient overflows.  FP32: the
 // hardware's reciprocal and a multiply, which is what a division is in the
 // FP32 build but for its rescaling of denominators above 2^96 (four more
 // instructions per quotient, of use only above 2^126, where the reciprocal is
@@ -142,7 +147,7 @@ struct Denom<double> {
   __device__ __forceinline__ Denom(double d, double inv) : b(d), r(inv) {}
   __device__ __forceinline__ double operator()(double a) const {
     const double q = a * r;
-    return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+    return __builtin_fma(-__builtin_fma(b, q, -a), r, q);
   }
 };
 
@@ -1195,15 +1200,18 @@ __device__ __forceinline__ void hllc_flux(const Consts& C, const MState<T>& L,
   const T* FK = left ? FL : FR;
   const T SK = left ? SL : SR, ptK = left ? ptL : ptR;
   const T sk = SK - K.u;
-  const Denom<T> by(SK - SM);
+  // left of the contact both sides of the quotients are negative: over a
+  // positive denominator a zero numerator gives the division's sign
+  const T sg = left ? T(-1) : T(1);
+  const Denom<T> by(sg * (SK - SM));
   T S[8];
-  S[0] = by(K.rho * sk);
+  S[0] = by(sg * (K.rho * sk));
   S[1] = S[0] * SM;
-  S[2] = by(K.rho * K.v * sk - c4 * (bx * hy - K.bx * K.by));
-  S[3] = by(K.rho * K.w * sk - c4 * (bx * bz - K.bx * K.bz));
-  S[4] = by(UK[4] * sk - ptK * K.u + ptS * SM +
-            c4 * (K.bx * (K.u * K.bx + K.v * K.by + K.w * K.bz) -
-                  bx * (SM * bx + vh * hy + wh * bz)));
+  S[2] = by(sg * (K.rho * K.v * sk - c4 * (bx * hy - K.bx * K.by)));
+  S[3] = by(sg * (K.rho * K.w * sk - c4 * (bx * bz - K.bx * K.bz)));
+  S[4] = by(sg * (UK[4] * sk - ptK * K.u + ptS * SM +
+                  c4 * (K.bx * (K.u * K.bx + K.v * K.by + K.w * K.bz) -
+                        bx * (SM * bx + vh * hy + wh * bz))));
   S[5] = bx; S[6] = hy; S[7] = bz;
 #pragma unroll
   for (int c = 0; c < 8; ++c) out[c] = FK[c] + SK * (S[c] - UK[c]);
