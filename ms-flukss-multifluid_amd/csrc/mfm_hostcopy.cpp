@@ -125,8 +125,9 @@ hipError_t host_copy(HostLink& link, void* dev, void* host, const CopySeg* seg, 
       (void)hipGetLastError();
     }
   }
-  HostCopier* hc = link.copier;
-  own = own && hc && hc->device == cur;
+  // (link.copier is the lock holder's to read: another thread may be making it)
+  HostCopier* hc = own ? link.copier : nullptr;
+  own = hc && hc->device == cur;
   char* d = static_cast<char*>(dev);
   char* p = static_cast<char*>(host);
   if (!own) {
