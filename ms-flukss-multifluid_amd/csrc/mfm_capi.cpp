@@ -1544,11 +1544,11 @@ int mfm_patch_update_host(mfm_ctx* c, mfm_fab U, mfm_box valid, double dt,
     const HBox v = hb(valid);
     const int top = dims - 1;
     const size_t plane = (size_t)ub.size() / (size_t)ub.n(top) * sizeof(double);
-    std::vector<CopySeg> seg((size_t)U.ncomp);
+    CopySeg seg[kMaxComp];  // (the update has accepted U.ncomp)
     for (int q = 0; q < U.ncomp; ++q)
       seg[q] = {((size_t)q * ub.n(top) + (size_t)(v.lo[top] - ub.lo[top])) * plane,
                 (size_t)v.n(top) * plane};
-    e = host_copy(c->link, dU, U.data, seg.data(), U.ncomp, false);
+    e = host_copy(c->link, dU, U.data, seg, U.ncomp, false);
     for (int d = 0; F && d < dims && e == hipSuccess; ++d)
       e = hipMemcpy(F[d].data, dF[d], (size_t)hb(F[d].box).size() * F[d].ncomp * sizeof(double),
                     hipMemcpyDeviceToHost);

@@ -15,9 +15,9 @@
 
 #include <algorithm>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 
 #include "mfm_host.hpp"
@@ -142,8 +142,8 @@ hipError_t host_copy(HostLink& link, void* dev, void* host, const CopySeg* seg, 
     auto body = [&, t]() { res[t] = hc->run(t, d, p, seg, nseg, to_dev); };
     try {
       th[t] = std::thread(body);
-    } catch (const std::system_error&) {
-      body();  // no thread to be had: its part here
+    } catch (const std::exception&) {
+      body();  // no thread to be had, or no memory for one: its part here
     }
   }
   res[0] = hc->run(0, d, p, seg, nseg, to_dev);

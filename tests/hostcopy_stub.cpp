@@ -3,12 +3,14 @@
 //   race:  eight threads copy through one link at a time, every copy checked
 //          (built with the thread sanitizer)
 //   pinned: memory that the runtime knows
+//   alloc: a thread that cannot be started for want of memory
 #include <hip/hip_runtime.h>
 
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -16,6 +18,18 @@
 
 static const void* pinned = nullptr;  // memory the runtime knows
 static std::atomic<int> whole_copies{0}, chunks{0};
+
+static thread_local int countdown = 0;  // the allocation that fails, 0: none
+
+#if !__has_feature(thread_sanitizer)  // (it brings its own)
+void* operator new(std::size_t n) {
+  if (countdown > 0 && --countdown == 0) throw std::bad_alloc();
+  if (void* p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, std::size_t) noexcept { std::free(p); }
+#endif
 
 extern "C" {
 hipError_t hipSetDevice(int) { return hipSuccess; }
@@ -76,6 +90,18 @@ int main(int argc, char** argv) {
     if (whole_copies != 1 || chunks != 0) ++bad;
     if (host_copy(link, dev.data(), other.data(), &all, 1, false) != hipSuccess) ++bad;
     if (whole_copies != 1 || chunks != 3 || std::memcmp(other.data(), host.data(), n)) ++bad;
+  } else if (argc > 1 && !std::strcmp(argv[1], "alloc")) {
+    HostLink link;
+    if (!round_trip(link, 1)) return 1;
+    for (int nth = 1; nth <= 4; ++nth) {  // of a copy's allocations
+      const size_t n = (size_t)6 << 20;
+      std::vector<char> host(n, (char)nth), dev(n);
+      const CopySeg all{0, n};
+      countdown = nth;
+      const hipError_t e = host_copy(link, dev.data(), host.data(), &all, 1, true);
+      countdown = 0;
+      if (e != hipSuccess || std::memcmp(host.data(), dev.data(), n)) ++bad;
+    }
   } else {
     for (int turn = 0; turn < 6; ++turn) {
       HostLink link;  // its first copy makes the pipeline, with others beside it

@@ -44,6 +44,13 @@ def test_pinned_memory_is_the_runtimes(tmp_path):
     assert r.returncode == 0 and "copies right" in r.stdout, r.stdout + r.stderr[:2000]
 
 
+def test_threads_that_do_not_start(tmp_path):
+    """A thread's own allocation fails: its part is copied by the caller, and
+    no exception leaves the C entry point."""
+    r = subprocess.run([build(tmp_path, []), "alloc"], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and "copies right" in r.stdout, r.stdout + r.stderr[:2000]
+
+
 @pytest.mark.gpu
 def test_threads_fetch_from_one_server():
     from test_serve import req_params, run_until_done
