@@ -270,7 +270,10 @@ int mfm_ctx_get_timing(mfm_ctx* ctx, int stage, int kind, double* ms,
  * face fluxes (RK2 with F stays separate), where they are the faster ones,
  * with shorter z-chunks (tz at most) for small
  * calls -- else the separate kernels; the allocation-free entry point always
- * takes the separate kernels.  AUTO decides per call: in the FP32-flux build
+ * takes the separate kernels, and so does a context whose scratch for the
+ * sums found no memory, until this function is called again (but for
+ * MFM_STAGE_SUMMED with FP32 fluxes, RK2 or first order: MFM_ERR_NOMEM).
+ * AUTO decides per call: in the FP32-flux build
  * a patch updated alone and in a level can then take different structures
  * (results equal within the FP32 bar, not bit for bit; the FP64 build gives
  * the same bits in both); a fixed mode gives the same bits whatever the

@@ -491,6 +491,7 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
   if (C0.char_rec || (han && mode == MFM_STAGE_FUSED) ||
       (fixed && mode == MFM_STAGE_SUMMED && (han || !f32)))
     mode = MFM_STAGE_SEPARATE;
+  if (separate) mode = MFM_STAGE_SEPARATE;
   const bool choose = mode == MFM_STAGE_AUTO;
   bool filled = false;  // the boxes fill 64 x 8 tiles
   int sum_block = f32 ? 512 : 256;
@@ -498,7 +499,7 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
   const int slots256 = sum_slots(256, f32 ? 4 : 8, C0.dedner);
   if (choose) {
     mode = MFM_STAGE_SEPARATE;
-    if (!fixed && !separate) {
+    if (!fixed) {
       TileCache t512{512, sum_slots(512, 4, 0), {}}, t256{256, slots256, {}};
       bool fluxes = false;
       double cells = 0.0, slots = 0.0, r512 = 0.0, r256 = 0.0, p512 = 0.0, p256 = 0.0;
@@ -721,10 +722,17 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
     A = fixed->dev;
     h = fixed->host;
   } else {
-    int rc = ensure_arena(c, off);
-    // the face sums take more scratch than the separate kernels
-    if (rc == MFM_ERR_NOMEM && choose && summed)
+    // The face sums take more scratch than the separate kernels, which run
+    // where it finds no memory (a fixed mode too, but for the FP32-flux build's,
+    // whose results are its own).  The context remembers the refusal: asked
+    // again, each call would free and allocate the scratch.
+    const bool either = summed && (choose || !f32 || han);
+    int rc = MFM_ERR_NOMEM;
+    if (!either || off <= c->arena_bytes || off < c->sums_refused) rc = ensure_arena(c, off);
+    if (rc == MFM_ERR_NOMEM && either) {
+      c->sums_refused = std::min(c->sums_refused, off);
       return run_batch(c, Ct, nct, in, n, new_dt, min_cell, level_dt, min_patch, s, fixed, true);
+    }
     if (rc) return rc;
     rc = ensure_hbuf(c, host_need);
     if (rc) return rc;
@@ -1315,6 +1323,7 @@ int mfm_ctx_set_stage_kernel(mfm_ctx* c, int mode, int tz) {
   if (mode < MFM_STAGE_SEPARATE || mode > MFM_STAGE_AUTO) return MFM_ERR_ARG;
   c->stage_mode = mode;
   c->stage_tz = tz;
+  c->sums_refused = std::numeric_limits<size_t>::max();
   return MFM_OK;
 }
 

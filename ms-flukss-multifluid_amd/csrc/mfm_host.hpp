@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <limits>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -38,6 +39,8 @@ struct mfm_ctx {
   mfm::host::HostLink link;
   double* host_u = nullptr;
   size_t host_u_bytes = 0;
+  // the least scratch that found no memory for the face sums
+  size_t sums_refused = std::numeric_limits<size_t>::max();
   bool host_busy = false;  // host_u is the state of a running update
   size_t fsize() const { return p.precision == MFM_PREC_FP32_FLUX ? 4 : 8; }
   // optional per-kernel timing, accumulated per stage and kernel kind
@@ -169,8 +172,8 @@ inline int tile_limiter(const Consts& C) {
   return C.plasma_lim == MFM_LIM_MINMOD || C.plasma_lim == MFM_LIM_VANLEER ? C.plasma_lim : -1;
 }
 
-// separate: MFM_STAGE_AUTO takes the separate kernels (too little memory for
-// the face sums' scratch).
+// separate: the separate kernels instead of the face sums, whose scratch found
+// no memory.
 int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
               double* new_dt, int* min_cell, double* level_dt, int* min_patch,
               hipStream_t s, const FixedScratch* fixed = nullptr, bool separate = false);
