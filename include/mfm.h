@@ -311,7 +311,7 @@ int mfm_patch_update_dev(mfm_ctx* ctx, mfm_fab U, mfm_box valid,
                          double* new_dt, int min_cell[3], void* stream);
 /* Same contract with host FABs: stages U (and F, divB) through HBM.  The
  * context keeps U's device memory for its next call (as large as the largest
- * U so far, given up when scratch memory needs it) and, once a U has 4 MiB,
+ * U so far, given up when scratch memory needs it or a call fails) and, once a U has 4 MiB,
  * 16 MiB of pinned copy buffers; both end with the context.               */
 int mfm_patch_update_host(mfm_ctx* ctx, mfm_fab U, mfm_box valid,
                           double dt, double dx, double time,

@@ -1569,6 +1569,11 @@ int mfm_patch_update_host(mfm_ctx* c, mfm_fab U, mfm_box valid, double dt,
   for (int d = 0; d < 3; ++d)
     if (dF[d]) (void)hipFree(dF[d]);
   if (dD) (void)hipFree(dD);
+  if (rc && rc != MFM_ERR_NUMERIC) {  // a call that failed keeps no memory
+    (void)hipFree(c->host_u);
+    c->host_u = nullptr;
+    c->host_u_bytes = 0;
+  }
   return rc;
 }
 

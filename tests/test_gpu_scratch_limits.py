@@ -95,3 +95,28 @@ def test_refused_sums():
     ctx.set_stage_kernel(mfmhd.STAGE_AUTO)
     assert step(ctx, patches[3])[0]
     ctx.close()
+
+
+def test_failed_host_call_keeps_no_memory():
+    """U finds device memory, its scratch does not: the call's U is given back,
+    and a smaller call fits."""
+    p = periodic_params(nf=NF)
+    nc = mfmhd.num_components(p)
+    vhi = tuple(n - 1 for n in N)
+    lo, hi, shape = grid_shape(nc, (0, 0, 0), vhi, 4)
+    U = periodic_fill(smooth_state(p, shape, lo, seed=1), 4)
+    slo, _, sshape = grid_shape(nc, (0, 0, 0), (19, 19, 19), 4)
+    V = periodic_fill(smooth_state(p, sshape, slo, seed=2), 4)
+    ctx = mfmhd.Context(p)
+    ctx.update_state_host(V, slo, mfmhd.Box.of((0, 0, 0), (19, 19, 19)), 2e-3, 1.0 / 32)
+    held = Held(U.nbytes + (512 << 20))
+    try:
+        before = free_bytes()
+        assert U.nbytes + (64 << 20) < before < scratch(nc, False)
+        with pytest.raises(mfmhd.MfmError):
+            ctx.update_state_host(U, lo, mfmhd.Box.of((0, 0, 0), vhi), 2e-3, 1.0 / 32)
+        assert free_bytes() > before - U.nbytes // 2
+        ctx.update_state_host(V, slo, mfmhd.Box.of((0, 0, 0), (19, 19, 19)), 2e-3, 1.0 / 32)
+    finally:
+        held.free()
+        ctx.close()
