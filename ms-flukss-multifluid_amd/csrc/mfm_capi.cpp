@@ -194,11 +194,18 @@ long tile_rounds(const Tile& t, int block) {
   auto rounds = [&](long f) { return (f + block - 1) / block; };
   return rounds((t.tx + 1L) * t.ty) + rounds(t.tx * (t.ty + 1L)) + rounds((long)t.tx * t.ty);
 }
+// Every width ceil(nx / kx) from the block's down to 16, each once: at most 500,
+// however long the box (20 us for both blocks; 0.5 us at 64, 5 at 1024 columns).
 Tile sum_tile(long nx, long ny, int block, int slots) {
   Tile best{1, 1};
   long cost = std::numeric_limits<long>::max();
-  for (long kx = 1; kx == 1 || kx <= nx / 16; ++kx) {
-    const long tx = std::min((nx + kx - 1) / kx, (long)block);
+  long last = 0;
+  for (long kx = 1, step; kx == 1 || kx <= nx / 16; kx = step) {
+    const long whole = (nx + kx - 1) / kx, tx = std::min(whole, (long)block);
+    // the next kx with a narrower tile
+    step = tx > 1 ? std::max(kx + 1, (nx + tx - 2) / (tx - 1)) : kx + 1;
+    if (tx == last) continue;
+    last = tx;
     const long most = std::min({(long)block / tx, (slots - tx) / (3 * tx + 1), ny});
     for (long ty = most; ty >= 1 && 2 * ty > most; --ty) {
       const Tile t{(int)tx, (int)ty};
@@ -496,35 +503,44 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
   bool filled = false;  // the boxes fill 64 x 8 tiles
   int sum_block = f32 ? 512 : 256;
   int tz = std::max(1, c->stage_tz);
-  const int slots256 = sum_slots(256, f32 ? 4 : 8, C0.dedner);
+  TileCache t512{512, sum_slots(512, 4, 0), {}},
+      t256{256, sum_slots(256, f32 ? 4 : 8, C0.dedner), {}};
   if (choose) {
     mode = MFM_STAGE_SEPARATE;
     if (!fixed) {
-      TileCache t512{512, sum_slots(512, 4, 0), {}}, t256{256, slots256, {}};
       bool fluxes = false;
-      double cells = 0.0, slots = 0.0, r512 = 0.0, r256 = 0.0, p512 = 0.0, p256 = 0.0;
-      for (int q = 0; q < n; ++q) {
-        if (in[q].cidx < 0 || in[q].cidx >= nct) continue;
-        const HBox v = clip(Ct[in[q].cidx], hb(in[q].valid));
-        if (v.size() <= 0) continue;
-        fluxes = fluxes || in[q].F;
+      double cells = 0.0, slots = 0.0;
+      auto boxes = [&](auto&& use) {
+        for (int q = 0; q < n; ++q) {
+          if (in[q].cidx < 0 || in[q].cidx >= nct) continue;
+          const HBox v = clip(Ct[in[q].cidx], hb(in[q].valid));
+          if (v.size() > 0) use(in[q], v);
+        }
+      };
+      boxes([&](const PatchIn& P, const HBox& v) {
+        fluxes = fluxes || P.F;
         cells += (double)v.size();
         slots += (double)((v.n(0) + 63) / 64 * 64) * (double)((v.n(1) + 7) / 8 * 8) * (double)v.n(2);
-        if (f32) sum_rounds(v, t512.of(v), 512, r512, p512);
-        sum_rounds(v, t256.of(v), 256, r256, p256);
-      }
+      });
       filled = slots > 0.0 && cells >= kAutoTileFill * slots;
       if (f32 && !han && filled) mode = MFM_STAGE_SUMMED;
       const bool one_lim = C0.plasma_lim == MFM_LIM_MINMOD || C0.plasma_lim == MFM_LIM_VANLEER;
       if (dims == 3 && one_lim && cells >= auto_cells(f32, p.time_approx, C0.nf, fluxes))
         mode = MFM_STAGE_SUMMED;
-      if (f32 && r256 < r512) sum_block = 256;
-      // shorter z-chunks where the blocks would not fill the chip
-      const double planes = sum_block == 512 ? p512 : 0.5 * p256;
-      while (tz > 1 && planes < kAutoBlocks * tz) tz /= 2;
+      if (mode == MFM_STAGE_SUMMED) {  // the block and the chunks (the search takes host time)
+        double r512 = 0.0, r256 = 0.0, p512 = 0.0, p256 = 0.0;
+        boxes([&](const PatchIn&, const HBox& v) {
+          if (f32) sum_rounds(v, t512.of(v), 512, r512, p512);
+          sum_rounds(v, t256.of(v), 256, r256, p256);
+        });
+        if (f32 && r256 < r512) sum_block = 256;
+        // shorter z-chunks where the blocks would not fill the chip
+        const double planes = sum_block == 512 ? p512 : 0.5 * p256;
+        while (tz > 1 && planes < kAutoBlocks * tz) tz /= 2;
+      }
     }
   }
-  TileCache tiles{sum_block, sum_block == 512 ? sum_slots(512, 4, 0) : slots256, {}};
+  TileCache& tiles = sum_block == 512 ? t512 : t256;
   const bool fused = mode == MFM_STAGE_FUSED;
   const bool summed = mode == MFM_STAGE_SUMMED;
   // FP32 fluxes: the face sums in FP64 where the call's other structure, the
