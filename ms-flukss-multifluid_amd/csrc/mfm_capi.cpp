@@ -912,7 +912,8 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
   if (c->graphs && !c->timer && !fixed) {
     // The kernels read every per-call value (dt, time, constants, tables)
     // from the arena, refreshed by the copy above; the sequence itself only
-    // depends on the arena layout and the list sizes.
+    // depends on the arena layout, the list sizes and where the directions of
+    // the face lists begin.
     std::vector<long long> key = {(long long)(uintptr_t)A, (long long)off_patch,
                                   (long long)off_ct, (long long)off_dtp, (long long)off_idp,
                                   (long long)off_dto, (long long)off_ido, dims, p.time_approx,
@@ -923,6 +924,11 @@ int run_batch(mfm_ctx* c, const Consts* Ct, int nct, const PatchIn* in, int n,
       key.push_back((long long)lists[l]->v.size());
       key.push_back((long long)lists[l]->nblk);
     }
+    for (const FaceBuilder* b : {&st1_flux, &st1_fbc, &st2_flux, &st2_fbc})
+      for (int d = 1; d < 4; ++d) {
+        key.push_back(b->f.reg[d]);
+        key.push_back(b->f.blk[d]);
+      }
     if (!c->gexec || key != c->gkey) {
       if (c->gexec) { (void)hipGraphExecDestroy(c->gexec); c->gexec = nullptr; }
       if (!c->cap_stream) {
