@@ -54,9 +54,10 @@ struct InterpArgs {
   double c_centre, c_side, dxc, dxf, coeff, tiny;
 };
 
-// Blocks of the rectangle copies: of: each block's rectangle.
-constexpr int kRectBlock = 64;
-hipError_t launch_rect_copy(const CopyRect* R, const int* of, int nblk,
+// Blocks of the rectangle copies: of: each block's rectangle; blk: their
+// threads, one of the two below.
+constexpr int kRectBlock = 64, kRectBlockLarge = 256;
+hipError_t launch_rect_copy(const CopyRect* R, const int* of, int nblk, int blk,
                             const FillFab* src_new, const FillFab* src_old,
                             const FillFab* dst, int nc, double a, double b,
                             int mode, hipStream_t s);
