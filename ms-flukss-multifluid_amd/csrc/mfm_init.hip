@@ -175,8 +175,11 @@ __global__ __launch_bounds__(kB) void k_init(Consts C, double* U, Geo G,
 // cell congruent to it modulo the box size.  blockIdx.y: a chunk of the
 // components, whose loads leave before its stores (the compiler may not move
 // a load of U across a store to it: one component at a time took a memory
-// latency each: 5.7 -> 4.7 us for 8 components of an 800-cell tube).
-constexpr int kPeriodicComps = 8;
+// latency each: 5.7 -> 4.7 us for 8 components of an 800-cell tube).  Where the
+// cells alone fill the chip a thread takes the chunks one after the other: most
+// threads have a cell that is no ghost and would only start and end (128^3, 23
+// components, 53 -> 42 us, 256^3 347 -> 226).
+constexpr int kPeriodicComps = 8, kPeriodicBlocks = 2048;
 __global__ __launch_bounds__(kB) void k_fill_periodic(double* U, Geo G, int nc,
                                                       int vlo0, int vlo1,
                                                       int vlo2, int vn0,
@@ -202,14 +205,15 @@ __global__ __launch_bounds__(kB) void k_fill_periodic(double* U, Geo G, int nc,
   if (!ghost) return;
   const long s = (long)(src[0] - G.ulo[0]) +
                  (long)G.un[0] * ((long)(src[1] - G.ulo[1]) + (long)G.un[1] * (src[2] - G.ulo[2]));
-  const int c0 = (int)blockIdx.y * kPeriodicComps;
-  double v[kPeriodicComps];
+  for (int c0 = (int)blockIdx.y * kPeriodicComps; c0 < nc; c0 += (int)gridDim.y * kPeriodicComps) {
+    double v[kPeriodicComps];
 #pragma unroll
-  for (int q = 0; q < kPeriodicComps; ++q)
-    if (c0 + q < nc) v[q] = U[s + (c0 + q) * G.ucs];
+    for (int q = 0; q < kPeriodicComps; ++q)
+      if (c0 + q < nc) v[q] = U[s + (c0 + q) * G.ucs];
 #pragma unroll
-  for (int q = 0; q < kPeriodicComps; ++q)
-    if (c0 + q < nc) U[t + (c0 + q) * G.ucs] = v[q];
+    for (int q = 0; q < kPeriodicComps; ++q)
+      if (c0 + q < nc) U[t + (c0 + q) * G.ucs] = v[q];
+  }
 }
 }  // namespace
 
@@ -233,9 +237,11 @@ hipError_t launch_fill_periodic(double* U, const int ulo[3], const int un[3],
   for (int d = 0; d < 3; ++d) { G.ulo[d] = ulo[d]; G.un[d] = un[d]; G.lo[d] = 0; G.n[d] = 0; }
   G.ucs = ucs;
   const long tot = (long)un[0] * un[1] * un[2];
+  const unsigned blocks = (unsigned)((tot + kB - 1) / kB);
   hipLaunchKernelGGL(k_fill_periodic,
-                     dim3((unsigned)((tot + kB - 1) / kB),
-                          (unsigned)((nc + kPeriodicComps - 1) / kPeriodicComps)),
+                     dim3(blocks, blocks >= (unsigned)kPeriodicBlocks
+                                      ? 1u
+                                      : (unsigned)((nc + kPeriodicComps - 1) / kPeriodicComps)),
                      dim3(kB), 0, s, U, G, nc, vlo[0], vlo[1], vlo[2], vn[0],
                      vn[1], vn[2], dims);
   return hipGetLastError();

@@ -1,11 +1,15 @@
 """Ghost copies of large boxes: rectangles whose mean size takes the exchange
-in large blocks, of one and several component chunks, in 3-D and 2-D."""
+in large blocks, and periodic fills of more than 2048 blocks, where a thread
+takes the component chunks one after the other; one and several chunks, in 3-D
+and 2-D."""
 import numpy as np
 import pytest
 
 import mfmhd
 from fill_layouts import grown, level_params, split
+from helpers import GpuPatch, grid_shape, periodic_fill
 from test_gpu_fill import same, to_dev
+from test_gpu_parity import periodic_params
 
 pytestmark = pytest.mark.gpu
 
@@ -36,4 +40,24 @@ def test_exchange_of_large_boxes(oracle_mod, dims, n, parts, nf):
     for d, a in zip(devs, arrs):
         assert same(d.numpy(), a)
     plan.close()
+    ctx.close()
+
+
+@pytest.mark.parametrize("dims,n,nf,ded", [
+    (3, (83, 79, 71), 4, True),       # 24 components, below 2048 blocks
+    (3, (91, 83, 89), 4, True),       # above
+    (3, (91, 83, 89), 1, False),
+    (2, (1021, 701, 1), 3, False),
+])
+def test_periodic_fill_of_large_boxes(dims, n, nf, ded):
+    print("large periodic fill", dims, n, nf, flush=True)
+    p = periodic_params(nf=nf, dims=dims, dedner=ded, eight=not ded)
+    nc = mfmhd.num_components(p)
+    vhi = tuple(v - 1 for v in n)
+    lo, hi, shape = grid_shape(nc, (0, 0, 0), vhi, 4, dims)
+    U = np.random.default_rng(nf).uniform(1, 2, shape)
+    g = GpuPatch(U, lo)
+    ctx = mfmhd.Context(p)
+    ctx.fill_periodic(g.fab, mfmhd.Box.of((0, 0, 0), vhi))
+    assert np.array_equal(g.numpy(), periodic_fill(U.copy(), 4, dims))
     ctx.close()
