@@ -1571,7 +1571,7 @@ int mfm_patch_update_host(mfm_ctx* c, mfm_fab U, mfm_box valid, double dt,
   }
   if (!rc || rc == MFM_ERR_NUMERIC) {
     // the update writes the valid box only: of each component, the planes
-    // that hold it come back
+    // that hold it come back (and, where one copy is cheaper, the rest as it was)
     const HBox v = hb(valid);
     const int top = dims - 1;
     const size_t plane = (size_t)ub.size() / (size_t)ub.n(top) * sizeof(double);
@@ -1579,7 +1579,7 @@ int mfm_patch_update_host(mfm_ctx* c, mfm_fab U, mfm_box valid, double dt,
     for (int q = 0; q < U.ncomp; ++q)
       seg[q] = {((size_t)q * ub.n(top) + (size_t)(v.lo[top] - ub.lo[top])) * plane,
                 (size_t)v.n(top) * plane};
-    e = host_copy(c->link, dU, U.data, seg, U.ncomp, false);
+    e = host_copy(c->link, dU, U.data, seg, U.ncomp, false, true);
     for (int d = 0; F && d < dims && e == hipSuccess; ++d)
       e = hipMemcpy(F[d].data, dF[d], (size_t)hb(F[d].box).size() * F[d].ncomp * sizeof(double),
                     hipMemcpyDeviceToHost);

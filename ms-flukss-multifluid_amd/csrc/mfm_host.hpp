@@ -183,9 +183,10 @@ struct CopySeg {
 };
 // Copies the segments between pageable (or pinned) host memory and the device,
 // large copies through the link's pinned buffers; returns when they are done.
-// Ordered after the null stream's work.
+// Ordered after the null stream's work.  The segments ascend; gaps_agree: both
+// sides hold the same bytes between them, which may be copied too.
 hipError_t host_copy(HostLink& link, void* dev, void* host, const CopySeg* seg, int nseg,
-                     bool to_dev);
+                     bool to_dev, bool gaps_agree = false);
 // Resolves, once per device, the address of the fixed scratch of the
 // allocation-free entry point on the context's device (mfm_noalloc.hip).
 int fixed_scratch_setup(mfm_ctx* c);

@@ -99,9 +99,26 @@ struct HostCopier {
 HostLink::~HostLink() { delete copier; }
 
 hipError_t host_copy(HostLink& link, void* dev, void* host, const CopySeg* seg, int nseg,
-                     bool to_dev) {
+                     bool to_dev, bool gaps_agree) {
   size_t total = 0;
   for (int s = 0; s < nseg; ++s) total += seg[s].bytes;
+  char* d = static_cast<char*>(dev);
+  char* p = static_cast<char*>(host);
+  // The runtime's copy: one of all the bytes from the first segment to the last
+  // where those between agree, else one per segment (a call takes several
+  // microseconds however little it copies).
+  auto runtime = [&]() -> hipError_t {
+    hipError_t r = hipSuccess;
+    const size_t all = seg[nseg - 1].off + seg[nseg - 1].bytes - seg[0].off;
+    const int m = gaps_agree ? 1 : nseg;
+    for (int s = 0; s < m && r == hipSuccess; ++s) {
+      const size_t bytes = gaps_agree ? all : seg[s].bytes;
+      r = to_dev ? hipMemcpy(d + seg[s].off, p + seg[s].off, bytes, hipMemcpyHostToDevice)
+                 : hipMemcpy(p + seg[s].off, d + seg[s].off, bytes, hipMemcpyDeviceToHost);
+    }
+    return r;
+  };
+  if (total < kLeast) return runtime();
   // what the null stream has queued comes first, as with a runtime copy
   hipError_t e = hipStreamSynchronize(nullptr);
   if (e != hipSuccess) return e;
@@ -115,7 +132,7 @@ hipError_t host_copy(HostLink& link, void* dev, void* host, const CopySeg* seg, 
   (void)hipGetLastError();  // (pageable memory may be reported as an error)
   // one copy at a time has the buffers; a second thread's is the runtime's
   std::unique_lock<std::mutex> lock(link.mu, std::defer_lock);
-  bool own = total >= kLeast && !known && lock.try_lock();
+  bool own = !known && lock.try_lock();
   if (own && !link.copier) {
     HostCopier* h = new (std::nothrow) HostCopier();
     if (h && h->open(cur) == hipSuccess) {
@@ -128,14 +145,7 @@ hipError_t host_copy(HostLink& link, void* dev, void* host, const CopySeg* seg, 
   // (link.copier is the lock holder's to read: another thread may be making it)
   HostCopier* hc = own ? link.copier : nullptr;
   own = hc && hc->device == cur;
-  char* d = static_cast<char*>(dev);
-  char* p = static_cast<char*>(host);
-  if (!own) {
-    for (int s = 0; s < nseg && e == hipSuccess; ++s)
-      e = to_dev ? hipMemcpy(d + seg[s].off, p + seg[s].off, seg[s].bytes, hipMemcpyHostToDevice)
-                 : hipMemcpy(p + seg[s].off, d + seg[s].off, seg[s].bytes, hipMemcpyDeviceToHost);
-    return e;
-  }
+  if (!own) return runtime();
   hipError_t res[kThreads];
   std::thread th[kThreads];
   for (int t = 1; t < kThreads; ++t) {

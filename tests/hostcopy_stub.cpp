@@ -3,9 +3,11 @@
 //   race:  eight threads copy through one link at a time, every copy checked
 //          (built with the thread sanitizer)
 //   pinned: memory that the runtime knows
+//   small: segments below the pipeline's size
 //   alloc: a thread that cannot be started for want of memory
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
@@ -90,6 +92,24 @@ int main(int argc, char** argv) {
     if (whole_copies != 1 || chunks != 0) ++bad;
     if (host_copy(link, dev.data(), other.data(), &all, 1, false) != hipSuccess) ++bad;
     if (whole_copies != 1 || chunks != 3 || std::memcmp(other.data(), host.data(), n)) ++bad;
+  } else if (argc > 1 && !std::strcmp(argv[1], "small")) {
+    HostLink link;
+    const size_t n = (size_t)1 << 20;
+    std::vector<char> host(n, 3), dev(n, 5);
+    const CopySeg seg[3] = {{100, 1000}, {5000, 70000}, {n - 50, 40}};
+    if (host_copy(link, dev.data(), host.data(), seg, 3, false) != hipSuccess) ++bad;
+    if (whole_copies != 3) ++bad;
+    for (size_t i = 0; i < n; ++i) {
+      bool in = false;
+      for (const CopySeg& s : seg) in = in || (i >= s.off && i < s.off + s.bytes);
+      if (host[i] != (in ? 5 : 3)) { ++bad; break; }
+    }
+    // the gaps may go along: one copy, nothing outside it
+    std::fill(host.begin(), host.end(), (char)3);
+    if (host_copy(link, dev.data(), host.data(), seg, 3, false, true) != hipSuccess) ++bad;
+    if (whole_copies != 4 || chunks != 0) ++bad;
+    for (size_t i = 0; i < n; ++i)
+      if (host[i] != (i >= 100 && i < n - 10 ? 5 : 3)) { ++bad; break; }
   } else if (argc > 1 && !std::strcmp(argv[1], "alloc")) {
     HostLink link;
     if (!round_trip(link, 1)) return 1;

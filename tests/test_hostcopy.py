@@ -39,8 +39,12 @@ def test_threads_share_one_link(tmp_path):
     assert "copies right" in r.stdout
 
 
-def test_pinned_memory_is_the_runtimes(tmp_path):
-    r = subprocess.run([build(tmp_path, []), "pinned"], capture_output=True, text=True, timeout=60)
+@pytest.mark.parametrize("program", ["pinned", "small"])
+def test_runtime_copies(tmp_path, program):
+    """Memory that the runtime knows, and copies below the pipeline's size: one
+    runtime copy where the bytes between the segments may go along (a small
+    state's components), else one per segment."""
+    r = subprocess.run([build(tmp_path, []), program], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and "copies right" in r.stdout, r.stdout + r.stderr[:2000]
 
 
