@@ -873,7 +873,7 @@ __device__ __forceinline__ void roe_flux(const Consts& C, const MState<T>& L,
 // are grouped by their shared factors, selects take the place of branches and
 // a reciprocal that several quotients share is formed once.  With the limiters
 // and quotients of this build (minmod32, Denom): 256^3, four fluids, the plasma's
-// tile kernel 1.29 -> 1.04 ms (720 -> 520 VALU instructions per face), the neutrals'
+// tile kernel 1.29 -> 1.04 ms (890 -> 650 VALU instructions per face), the neutrals'
 // 1.33 -> 1.19, a step 11.9 -> 11.2 ms; 91 x 75 x 53, two fluids, van Leer, the face
 // kernel 39 -> 24 us.  Errors against the FP64 flux over random states (smooth, jumps,
 // Mach 20, cold, without tangential field) equal the ungrouped form's.
